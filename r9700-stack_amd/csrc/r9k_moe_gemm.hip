@@ -464,6 +464,8 @@ int r9k_prefill_launch(long a, long as, long wq, long ws, long c, long sorted_id
                        long topk_w, long ws_estride, int max_blocks, int numel, int a_row_div, int K, int N,
                        long stream);
 int r9k_prefill_block_rows();
+int r9k_mid_launch(long a, long as, long wq, long ws, long c, long sorted_ids, long expert_ids, long ntpp, long topk_w,
+                   long ws_estride, int max_blocks, int numel, int a_row_div, int K, int N, int blk, long stream);
 int r9k_nvfp4_prefill_launch(long a, long as, long wq, long ws, long wg, long c, long sorted_ids, long expert_ids,
                              long ntpp, long topk_w, long ws_estride, long wg_estride, int max_blocks, int numel,
                              int a_row_div, int K, int N, int blk, long stream);
@@ -527,6 +529,11 @@ extern "C" int r9k_moe_4bit_prefill(int nv, long a, long as, long wq, long ws, l
   if (kPf[cfg].BM == r9k_prefill_block_rows() && K % 128 == 0 && getenv_flag_off("R9K_PREFILL_LDS") == 0)
     return r9k_prefill_launch(a, as, wq, ws, c, sorted_ids, expert_ids, ntpp, topk_w, ws_estride, max_blocks, numel,
                               a_row_div, K, N, stream);
+  // 64- and 128-row blocks, any K: the LDS-ring kernel (r9k_moe_mid.hip); what it does not address (2 GiB and more,
+  // unaligned bases), and 256-row blocks of other K, run on the decode kernel
+  const int mid = r9k_mid_launch(a, as, wq, ws, c, sorted_ids, expert_ids, ntpp, topk_w, ws_estride, max_blocks, numel,
+                                 a_row_div, K, N, kPf[cfg].BM, stream);
+  if (mid != 2) return mid;
   const int rc = moe_dispatch(a, as, wq, ws, c, sorted_ids, expert_ids, ntpp, topk_w, ws_estride, max_blocks, numel,
                               a_row_div, K, N, 4, kPf[cfg].BM, stream);
   if (rc) return rc;

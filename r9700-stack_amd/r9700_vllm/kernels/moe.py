@@ -444,16 +444,52 @@ def moe_gemm(a_q: torch.Tensor, a_s: torch.Tensor, w: Mxfp4Experts, out: torch.T
     return out
 
 
+# Dense MXFP4 linears on the 64- / 128-row LDS-ring kernel (r9k_moe_mid.hip, prefill cfgs MID_CFG / MID_CFG_BIG).
+# Below PREFILL_MIN_M rows it takes a step from DENSE_MID_M rows, earlier the more weight there is to stream per launch
+# (N * K): the decode kernel reads the activations once per wave, which costs little on a small weight. Measured on
+# MI355X, decode kernel (or r9k_dense_mxfp4_a8 up to 16 rows) -> this one, us: [17408, 5120] M = 4 / 6 / 16 / 32 / 48
+# 12.6 / 13.5 / 16.8 / 19.6 / 23.7 -> 12.9 / 12.8 / 12.8 / 13.3 / 14.8; [4096, 4096] M = 32 / 40 / 64 8.8 / 10.2 / 12.7
+# -> 10.4 / 9.8 / 9.7; [2048, 5120] M = 32 / 40 11.2 / 11.4 -> 11.0 / 10.5; [1024, 2048] M = 48 / 64 6.0 / 8.4 -> 7.1.
+MID_CFG, MID_CFG_BIG = 17, 10
+DENSE_MID_M = ((6, 1 << 25), (33, 1 << 23), (49, 0))           # (rows from, N * K from)
+_PREFILL_FORCED = "R9K_PREFILL_CFG" in os.environ or "R9K_PREFILL_CFG_SMALL" in os.environ
+
+
+def dense_mid_wanted(M: int, N: int, K: int) -> bool:
+    """Whether a dense MXFP4 linear of M < PREFILL_MIN_M rows runs on the LDS-ring kernel's 64-row blocks."""
+    return N % 16 == 0 and K % GROUP == 0 and any(M >= m and N * K >= nk for m, nk in DENSE_MID_M)
+
+
+def dense_prefill_cfg(M: int, N: int, K: int) -> int:
+    """Prefill tile of a dense MXFP4 linear from PREFILL_MIN_M rows, by the time its tiles take in units of one 128-wide
+    K step. The 256-row kernel runs one 256 x 256 tile a CU at 1.35 us a step, so whole rounds of 256 tiles; the 128-row
+    blocks run two 128 x 128 tiles a CU, 0.9 us a step for 512 of them (0.5 us when there are fewer than one a CU:
+    then 64-row blocks, whose tiles are smaller and split K). Measured on MI355X, 256-row -> 128- or 64-row blocks, us:
+    [17408, 5120] M = 511 / 700 / 1024 / 1500 / 2048 / 4096 55 / 56 / 111 / 111 / 170 / 285 against 50 / 63 / 82 / 113 /
+    148 / 297; [4096, 4096] M = 1024 / 2048 / 4096 43 / 45 / 54 against 20 / 31 / 57; [2048, 5120] 54-55 against 20 / 23 /
+    37; [640, 2560] M = 2048 29 against 13."""
+    if _PREFILL_FORCED:
+        return PREFILL_DEFAULT if M >= 512 else PREFILL_DEFAULT_SMALL
+    t128 = -(-M // 128) * -(-N // 128)
+    t256 = -(-M // 256) * -(-N // 256)
+    if K % 128 == 0 and M >= 256 and 1.35 * -(-t256 // 256) < max(0.5, 0.9 * t128 / 512):
+        return PREFILL_DEFAULT
+    return MID_CFG_BIG if t128 >= 256 else MID_CFG
+
+
 def pick_cfg(N: int, K: int, group: int = GROUP, M: int | None = None, kind: str | None = None,
              fold: bool = False) -> tuple:
-    """("P", cfg) for the prefill entry at M >= PREFILL_MIN_M, else the decode kernel's (WV, SK, NPW) launch shape on
+    """("P", cfg) for the prefill entry at M >= PREFILL_MIN_M (dense_prefill_cfg) and at the wider decode widths the
+    LDS-ring kernel takes (dense_mid_wanted), else the decode kernel's (WV, SK, NPW) launch shape on
     this device for a dense [M, K] x [N, K]^T product: the gfx950 table's entry (kernels/tuned.json, written by
     kernels/tune.py's sweep; WV = K-tiles per load batch, SK = waves splitting K, NPW = column tiles per wave) for the
     nearest measured M, or (0, 0, 0) -- the kernel's own choice -- for a shape the table does not hold.
     R9K_TUNED=0 ignores the table."""
     if kind and M:
         if M >= PREFILL_MIN_M and K % prefill_bk(PREFILL_DEFAULT) == 0:
-            return ("P", PREFILL_DEFAULT if M >= 512 else PREFILL_DEFAULT_SMALL)
+            return ("P", dense_prefill_cfg(M, N, K))
+        if M > DENSE_A8_MAX_M and dense_mid_wanted(M, N, K):
+            return ("P", MID_CFG)
     from . import tuned
     cfg = tuned.lookup(kind or "mxfp4", N, K, M or 1)
     return legal_cfg(cfg, N, K, group, decode_mt(M or 1)) if cfg else (0, 0, 0)
@@ -528,6 +564,32 @@ def pick_moe_prefill_block(numel: int, num_experts: int, K1: int, K2: int):
 # blocks, uniform routing at ~21 rows 6% slower.
 DEVICE_BLOCKS_MIN = int(os.environ.get("R9K_MOE_DEVICE_BLOCKS_MIN", "1024"))
 DEVICE_MIN_ROWS = int(os.environ.get("R9K_MOE_DEVICE_MIN_ROWS", "22"))
+
+
+# Routed steps of small experts (gate_up codes below SPLIT_DECODE_MIN_BYTES) from MID_MIN_ROWS rows an expert run on
+# 64-row blocks of the LDS-ring kernel, from MID_BIG_ROWS on 256-row blocks (128-row ones where a K is not a multiple of
+# 128), all without splitting the tables: a 64-row block streams its expert's weights once, so experts with a handful
+# of rows cost little more than their weights. Measured on MI355X, whole layer, us: 288 experts, hidden 2048, intermediate
+# 512, T = 600 / 1024 / 2048 / 4096: 206 / 222 / 225 / 273 on split tables, 189 / 189 / 202 / 250 on 256-row blocks, 183 /
+# 158 / 191 / 287 on 64-row ones (under Zipf(1.1) routing 139 / 140 / 183 / 253, 150 / 138 / 178 / 250 and 142 / 123 / 172
+# / 267); 512 experts, top-10, hidden 2560, intermediate 320 (GEMMs alone): T = 500 / 1000 / 1600 decode blocks 165 / 217 /
+# 299, 64-row blocks 155 / 163 / 176; T = 4096 (80 rows an expert) 64-row 307, 128-row 243.
+MID_MIN_ROWS, MID_BIG_ROWS = 10, 64
+
+
+def pick_mid_block(numel: int, num_experts: int, K1: int, K2: int):
+    """(cfg, rows per routing block) for a routed MXFP4 step on the LDS-ring kernel, else None."""
+    per = numel / max(1, min(num_experts, numel))
+    if per < MID_MIN_ROWS or not small_experts(K1, K2):
+        return None
+    if per < MID_BIG_ROWS:
+        return MID_CFG, prefill_block(MID_CFG)
+    return (MID_CFG_BIG, prefill_block(MID_CFG_BIG)) if K1 % 128 or K2 % 128 else None
+
+
+def small_experts(K1: int, K2: int) -> bool:
+    """Experts with fewer than SPLIT_DECODE_MIN_BYTES of gate_up codes (K1 * 2 K2 / 2 bytes)."""
+    return K1 * K2 < SPLIT_DECODE_MIN_BYTES
 
 
 def big_block_cfg(K1: int, K2: int):

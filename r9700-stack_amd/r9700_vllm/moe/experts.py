@@ -246,7 +246,16 @@ class R9700Mxfp4Experts(_experts_base()):
                 # experts split theirs) and for which it should build both layouts (route.dual_wanted)
                 layer._r9k_split_k = (K1, K2) if plain else None
                 layer._r9k_dual_blk = bc[1] if dual_ok else 0
-            split = plain and K.split_wanted(numel, E, K1, K2)
+            # the LDS-ring kernel's 64- / 128-row blocks (small experts), unless the router built this step's tables
+            mid = K.pick_mid_block(numel, E, K1, K2) if plain and not K.down_sum_fits(numel, N2, K2) else None
+            if mid is not None and route.take(layer, topk_ids, blk, numel) is not None:
+                mid = None
+            split = (plain and mid is None and K.split_wanted(numel, E, K1, K2)
+                     and not (big is not None and K.small_experts(K1, K2)))
+            if mid is not None:
+                pf_gate = pf_down = mid[0]
+                blk = mid[1]
+                dual_ok = False
             tabs = route.take(layer, topk_ids, blk, numel) if expert_map is None and not split else None
             tabs_big = route.take_big(layer, topk_ids, blk, numel) if tabs is not None else None
             tabs_small = None

@@ -84,7 +84,9 @@ def _mxfp4_linear_rows(x: torch.Tensor, W, out: torch.Tensor, fold: bool) -> Non
     if M <= KM.DENSE_QA_MAX_M and not fold and KM.dense_mxfp4_qa(x, W, out):   # decode widths: quant in the launch
         return
     q, s = KM.quant_rows_fp8(x)
-    mxfp4_gemm_q(q, s, W, out, M, KM.pick_cfg(W.N, W.K, M=M, kind="mxfp4", fold=fold))
+    cfg = ("P", KM.MID_CFG) if M < KM.PREFILL_MIN_M and KM.dense_mid_wanted(M, W.N, W.K) else (
+        KM.pick_cfg(W.N, W.K, M=M, kind="mxfp4", fold=fold))
+    mxfp4_gemm_q(q, s, W, out, M, cfg)
 
 
 def _mxfp4_linear(x: torch.Tensor, wq: torch.Tensor, wsr: torch.Tensor, N: int, K: int, fold: bool = False
