@@ -259,6 +259,12 @@ int r9k_dense_nvfp4_qa(long x, long ldx, long wq, long ws, long wg, long out, lo
  * [N][K/2], out_e8m0 u8 [N][K/32] (checkpoint layout). -2 K % 32, -3 bad pointer / alignment, -6 launch error. */
 int r9k_nvfp4_to_mxfp4(long packed, long s16, long row_div, long out_packed, long out_e8m0, int N, int K, long stream);
 
+/* Checkpoint MXFP4 weights to the kernels' layout in one launch: packed u8 [E][N][K/2] -> wq (the same bytes in fragment
+ * order), scale e8m0 u8 [E][N][K/32] -> ws u8 [E][K/32 + 1][N] (fragment order, then the per-row maximum). Either half is
+ * left out when its source is 0. wq must not overlap packed; codes 16-byte aligned, ws 4-byte. -1 N % 16, -2 K % 32,
+ * -3 bad pointer / alignment / E > 65535, -6 launch error. */
+int r9k_mxfp4_prep(long packed, long scale, long wq, long ws, int E, int N, int K, long stream);
+
 /* The same MSE search on fp32 weights [N][K] (r9700_vllm/quant/nvfp4.py:54-75, quantize_mxfp4_search). */
 int r9k_quantize_mxfp4_search(long w, long out_packed, long out_e8m0, int N, int K, long stream);
 

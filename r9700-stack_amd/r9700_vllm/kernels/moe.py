@@ -74,6 +74,8 @@ def lib() -> ctypes.CDLL:
         L.r9k_nvfp4_to_mxfp4.argtypes = [l] * 5 + [i] * 2 + [l]
         L.r9k_quantize_mxfp4_search.restype = i
         L.r9k_quantize_mxfp4_search.argtypes = [l] * 3 + [i] * 2 + [l]
+        L.r9k_mxfp4_prep.restype = i
+        L.r9k_mxfp4_prep.argtypes = [l] * 4 + [i] * 3 + [l]
         L.r9k_fold_supported.restype = i
         L.r9k_moe_down_sum.restype = i
         L.r9k_dense_mxfp4_qa.restype = i
@@ -167,6 +169,24 @@ def prepare_nvfp4_weights(packed: torch.Tensor, scale16: torch.Tensor, row_mult:
     return Nvfp4Experts(wq.view(torch.int32), ws, row_mult.float().reshape(E, N).contiguous(), N, K)
 
 
+def _prep_kernel(packed: torch.Tensor | None, scale: torch.Tensor | None, wq: torch.Tensor | None,
+                 wsr: torch.Tensor | None) -> bool:
+    """permute_fragments and / or pack_scales in one launch (r9k_mxfp4_prep) for contiguous, aligned tensors on the
+    current GPU; False (nothing launched) for anything else: the torch expressions then do it."""
+    ts = [t for t in (packed, scale, wq, wsr) if t is not None]
+    src = packed if packed is not None else scale
+    E, N, cols = src.shape
+    K = cols * (2 if packed is not None else GROUP)
+    if not (all(t.is_cuda and t.is_contiguous() and t.device.index == torch.cuda.current_device() for t in ts)
+            and N % 16 == 0 and K % GROUP == 0 and 0 < E <= 65535 and K > 0
+            and all(t.data_ptr() % 16 == 0 for t in (packed, wq) if t is not None)
+            and (wsr is None or wsr.data_ptr() % 4 == 0)):
+        return False
+    ptr = [t.data_ptr() if t is not None else 0 for t in (packed, scale, wq, wsr)]
+    _check(lib().r9k_mxfp4_prep(*ptr, E, N, K, _stream()), f"r9k_mxfp4_prep E={E} N={N} K={K}")
+    return True
+
+
 def permute_fragments(packed: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """[E, N, K/2] uint8 checkpoint order -> [E, N*K/8] int32 fragment order (same bytes, same size); written into
     `out` (any tensor of E * N * K/2 bytes, not overlapping `packed`) when given.
@@ -181,6 +201,8 @@ def permute_fragments(packed: torch.Tensor, out: torch.Tensor | None = None) -> 
     nt, nkf, G = N // 16, K // KTILE, (K % KTILE) // GROUP
     if out is None:
         out = torch.empty((E, N * Kh // 4), dtype=torch.int32, device=packed.device)
+    if packed.dtype == torch.uint8 and _prep_kernel(packed, None, out, None):
+        return out.view(torch.uint8).reshape(E, -1).view(torch.int32)
     dst = out.view(torch.uint8).reshape(E, nt, 8 * K)
     w = packed.reshape(E, nt, 16, Kh)
     if nkf:
@@ -213,7 +235,13 @@ def prepare_mxfp4_weights(packed: torch.Tensor, scale: torch.Tensor) -> Mxfp4Exp
     K = Kh * 2
     assert N % 16 == 0 and K % GROUP == 0, (N, K)
     assert scale.shape == (E, N, K // GROUP), (scale.shape, (E, N, K // GROUP))
-    return Mxfp4Experts(permute_fragments(packed.view(torch.uint8)), pack_scales(scale), N, K)
+    packed, scale = packed.view(torch.uint8), scale.view(torch.uint8)
+    if packed.is_cuda and packed.device == scale.device:
+        wq = torch.empty((E, N * Kh // 4), dtype=torch.int32, device=packed.device)
+        wsr = torch.empty((E, K // GROUP + 1, N), dtype=torch.uint8, device=packed.device)
+        if _prep_kernel(packed, scale, wq, wsr):
+            return Mxfp4Experts(wq, wsr, N, K)
+    return Mxfp4Experts(permute_fragments(packed), pack_scales(scale), N, K)
 
 
 def pack_scales(scale: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -228,6 +256,8 @@ def pack_scales(scale: torch.Tensor, out: torch.Tensor | None = None) -> torch.T
     nt, nkf, G = N // 16, KB // 4, KB % 4
     if out is None:
         out = torch.empty((E, KB + 1, N), dtype=torch.uint8, device=scale.device)
+    if out.dtype == torch.uint8 and _prep_kernel(None, scale, None, out):
+        return out
     body = out.view(E, -1)[:, : KB * N].view(E, nt, 16 * KB)
     s = scale.reshape(E, nt, 16, KB)                                                     # [E, nt, r, kb]
     if nkf:
