@@ -16,6 +16,27 @@ constexpr size_t NT_STREAM_BYTES = size_t(64) << 20;
 
 __device__ __forceinline__ float bf2f(uint16_t u) { return __uint_as_float((uint32_t)u << 16); }
 
+// n / d for 32-bit unsigned n by a divisor fixed per launch, as a multiply-high and shifts (Granlund & Montgomery,
+// "Division by invariant integers using multiplication", 1994, fig. 4.1): with l = ceil(log2 d) and
+// m = floor(2^32 (2^l - d) / d) + 1, n / d = (t + ((n - t) >> 1)) >> (l - 1), t = mulhi(n, m); l = 0 means d = 1.
+struct DivMagic {
+  uint32_t m;
+  int l;
+};
+
+inline DivMagic div_magic(uint32_t d) {
+  int l = 0;
+  while ((1ull << l) < d) l++;
+  const uint64_t m = ((1ull << 32) * ((1ull << l) - d)) / d + 1;
+  return {(uint32_t)m, l};
+}
+
+__device__ __forceinline__ uint32_t div_by(uint32_t n, DivMagic dm) {
+  if (dm.l == 0) return n;
+  const uint32_t t = __umulhi(n, dm.m);
+  return (t + ((n - t) >> 1)) >> (dm.l - 1);
+}
+
 // fp32 -> bf16, round to nearest even; NaN stays a quiet NaN (torch's conversion).
 __device__ __forceinline__ uint16_t f2bf(float f) {
   uint32_t u = __float_as_uint(f);

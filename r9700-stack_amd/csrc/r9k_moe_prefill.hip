@@ -46,27 +46,6 @@ struct __align__(16) Stage {
 };
 constexpr size_t SMEM = sizeof(Stage) * NSTAGE;
 
-// n / d for 32-bit unsigned n by a divisor fixed per launch, as a multiply-high and shifts (Granlund & Montgomery,
-// "Division by invariant integers using multiplication", 1994, fig. 4.1): with l = ceil(log2 d) and
-// m = floor(2^32 (2^l - d) / d) + 1, n / d = (t + ((n - t) >> 1)) >> (l - 1), t = mulhi(n, m); l = 0 means d = 1.
-struct DivMagic {
-  uint32_t m;
-  int l;
-};
-
-DivMagic div_magic(uint32_t d) {
-  int l = 0;
-  while ((1ull << l) < d) l++;
-  const uint64_t m = ((1ull << 32) * ((1ull << l) - d)) / d + 1;
-  return {(uint32_t)m, l};
-}
-
-__device__ __forceinline__ uint32_t div_by(uint32_t n, DivMagic dm) {
-  if (dm.l == 0) return n;
-  const uint32_t t = __umulhi(n, dm.m);
-  return (t + ((n - t) >> 1)) >> (dm.l - 1);
-}
-
 // 1 when the environment variable is set to "0" (a switch turned off).
 int getenv_flag_off_pf(const char* name) {
   const char* v = getenv(name);
