@@ -3,7 +3,7 @@
     python r9700-stack_amd/build.py            # -> r9700-stack_amd/r9700_vllm/kernels/libr9k.so
 
 Every `csrc/*.hip` is compiled for gfx950 only and linked into one shared library exporting the C-ABI declared in
-include/r9k.h. Objects go to `_build/` next to this file (not tracked).
+include/r9k.h, and the bindings' launch helpers (csrc/host) become `_r9k_launch.so` beside it. Objects go to `_build/` next to this file (not tracked).
 """
 from __future__ import annotations
 
@@ -17,6 +17,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "r9700_vllm", "kernels", "libr9k.so")
+LAUNCH = os.path.join(HERE, "r9700_vllm", "kernels", "_r9k_launch.so")
 BUILD = os.path.join(HERE, "_build")
 
 ARCH = "gfx950"
@@ -48,13 +49,35 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_launch(out: str = LAUNCH) -> str:
+    """The bindings' launch helpers (csrc/host/r9k_launch.cpp): a CPython extension over torch's C++ API, host code only."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"]]
+    lib = os.path.join(root, "lib")
+    tmp = out + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in inc),
+           os.path.join(CSRC, "host", "r9k_launch.cpp"), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-o", tmp]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode:
+        raise RuntimeError(f"g++ failed for r9k_launch.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, out)
+    return out
+
+
 def build(out: str = OUT, jobs: int = 8, verbose: bool = True) -> str:
     os.makedirs(BUILD, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
     if not srcs:
         raise RuntimeError(f"no HIP sources in {CSRC}")
-    with cf.ThreadPoolExecutor(max_workers=max(1, min(jobs, len(srcs)))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=max(1, min(jobs, len(srcs) + 1))) as ex:
+        launch = ex.submit(build_launch)
         objs = list(ex.map(_compile, srcs))
+        launch.result()
     tmp = out + ".tmp"
     cmd = [hipcc(), "-shared", f"--offload-arch={ARCH}", "-fPIC", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -1,0 +1,107 @@
+// r9k_launch.cpp -- the Python bindings' launch helpers as a CPython extension (r9700_vllm/kernels/_r9k_launch.so):
+//
+//   call(address, *args) -> int      a libr9k C entry: a tensor passes its data pointer, None 0, an int its value
+//   empty(like, dtype, *sizes)       torch.empty(sizes) of a torch.dtype on like's device
+//
+// A decode step is a handful of launches of a few microseconds, and its host side was bound by the bindings: a ctypes
+// call converts each argument by its argtype (a 20-argument launch with its data_ptr() calls ~5 us beside the ~3 us the
+// launch itself takes), torch.empty 1.7 us an output. Measured on MI355X's host, Python loop over one entry: see the
+// figures in kernels/moe.py. Entries with a floating-point argument stay on ctypes.
+//
+// Every libr9k entry takes long and int arguments only and returns int. They are called here through a type of as many
+// longs as arguments were given: on x86-64 an int parameter is the low half of the same register or stack slot.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <utility>
+
+#if !defined(__x86_64__)
+#error "the calling convention above is x86-64's"
+#endif
+
+namespace {
+
+constexpr int MAX_ARGS = 28;
+
+template <size_t>
+using Long = long;
+
+template <size_t... I>
+int call_n(long fn, const long* v, std::index_sequence<I...>) {
+  return reinterpret_cast<int (*)(Long<I>...)>(fn)(v[I]...);
+}
+
+template <size_t N>
+int dispatch(size_t n, long fn, const long* v) {
+  if (n == N) return call_n(fn, v, std::make_index_sequence<N>{});
+  if constexpr (N < MAX_ARGS) return dispatch<N + 1>(n, fn, v);
+  return -1000;
+}
+
+PyObject* py_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs < 2 || nargs - 1 > MAX_ARGS) {
+    PyErr_Format(PyExc_TypeError, "call(address, *args): 1 to %d arguments, got %zd", MAX_ARGS, nargs - 1);
+    return nullptr;
+  }
+  const long fn = PyLong_AsLong(args[0]);
+  if (fn == -1 && PyErr_Occurred()) return nullptr;
+  if (fn == 0) {
+    PyErr_SetString(PyExc_ValueError, "call: null entry address");
+    return nullptr;
+  }
+  long v[MAX_ARGS];
+  for (Py_ssize_t i = 1; i < nargs; i++) {
+    PyObject* a = args[i];
+    if (PyLong_Check(a)) {
+      v[i - 1] = PyLong_AsLong(a);
+      if (v[i - 1] == -1 && PyErr_Occurred()) return nullptr;
+    } else if (a == Py_None) {
+      v[i - 1] = 0;
+    } else if (THPVariable_Check(a)) {
+      v[i - 1] = reinterpret_cast<long>(THPVariable_Unpack(a).data_ptr());
+    } else {
+      PyErr_Format(PyExc_TypeError, "call: argument %zd is a %s, not an int, a tensor or None", i, Py_TYPE(a)->tp_name);
+      return nullptr;
+    }
+  }
+  return PyLong_FromLong(dispatch<1>((size_t)nargs - 1, fn, v));
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs < 3 || nargs > 6 || !THPVariable_Check(args[0]) || !THPDtype_Check(args[1])) {
+    PyErr_SetString(PyExc_TypeError, "empty(like, dtype, *sizes): a tensor, a torch.dtype and 1 to 4 ints");
+    return nullptr;
+  }
+  const at::Tensor& like = THPVariable_Unpack(args[0]);
+  int64_t sz[4];
+  for (Py_ssize_t i = 2; i < nargs; i++) {
+    sz[i - 2] = PyLong_AsLong(args[i]);
+    if (sz[i - 2] == -1 && PyErr_Occurred()) return nullptr;
+  }
+  return THPVariable_Wrap(at::empty(at::IntArrayRef(sz, (size_t)nargs - 2),
+                                    at::TensorOptions().dtype(reinterpret_cast<THPDtype*>(args[1])->scalar_type)
+                                        .device(like.device())));
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef kMethods[] = {
+    {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_call)), METH_FASTCALL,
+     "call(address, *args) -> int: a libr9k entry on tensors (their data pointers), ints and None (0)"},
+    {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_empty)), METH_FASTCALL,
+     "empty(like, dtype, *sizes) -> an uninitialised tensor on like's device"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_r9k_launch", "Launch helpers of the libr9k bindings.", -1, kMethods,
+                       nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__r9k_launch(void) { return PyModule_Create(&kModule); }

@@ -34,10 +34,19 @@ def table() -> dict:
     return _TABLE
 
 
+_INDEX: tuple = (None, {})            # (the table it was built from, {(kind, N, K): entries by ascending M})
+
+
 def lookup(kind: str, N: int, K: int, M: int):
     """(WV, SK, NPW) for this product, or None."""
-    rows = sorted((e for e in table().get("entries", ()) if e["kind"] == kind and e["N"] == N and e["K"] == K),
-                  key=lambda e: e["M"])
+    global _INDEX
+    tab = table()
+    if _INDEX[0] is not tab:
+        by: dict = {}
+        for e in sorted(tab.get("entries", ()), key=lambda e: e["M"]):
+            by.setdefault((e["kind"], e["N"], e["K"]), []).append(e)
+        _INDEX = (tab, by)
+    rows = _INDEX[1].get((kind, N, K))
     if not rows:
         return None
     best = rows[0]

@@ -39,16 +39,26 @@ MOE_FUSE = os.environ.get("R9K_MOE_FUSE", "0") == "1"
 BUF_LIMIT = (1 << 31) - 1
 
 
+def bytes_per_token(topk: int, N1: int, K1: int, N2: int, K2: int) -> int:
+    """The largest per-step buffer's bytes for one token (chunk_tokens)."""
+    return max(topk * N1 * 2, topk * N2 * 2, K1, topk * K2, topk * 4)
+
+
 def chunk_tokens(M: int, topk: int, N1: int, K1: int, N2: int, K2: int, limit: int = BUF_LIMIT) -> list:
     """Token ranges [(t0, t1), ...] covering 0..M, as few and as even as possible, such that in each range every
     per-step buffer stays <= `limit` bytes: the gate_up output [rows*topk, N1] and the down output [rows*topk, N2]
     (bf16), the fp8 activations of both GEMMs ([rows, K1] and [rows*topk, K2]) and the fp32 row scales."""
-    per_token = max(topk * N1 * 2, topk * N2 * 2, K1, topk * K2, topk * 4)
+    per_token = bytes_per_token(topk, N1, K1, N2, K2)
     n = -(-M // max(1, limit // per_token))
     if n == 0:
         return []
     bounds = [M * i // n for i in range(n + 1)]
     return list(zip(bounds[:-1], bounds[1:]))
+
+
+def _flat(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """t's values as one contiguous row of `dtype` (t itself, in its shape, when it is already contiguous)."""
+    return t if t.dtype == dtype and t.is_contiguous() else t.reshape(-1).to(dtype).contiguous()
 
 
 # A pass whose GEMMs run on the block stream (r9k_moe_stream over 16-row blocks): the small-expert table of a split
@@ -187,9 +197,8 @@ class R9700Mxfp4Experts(_experts_base()):
         if M == 0:
             return
 
-        chunks = chunk_tokens(M, topk, N1, K1, N2, K2)
-        if len(chunks) > 1:
-            for t0, t1 in chunks:
+        if M * bytes_per_token(topk, N1, K1, N2, K2) > BUF_LIMIT:
+            for t0, t1 in chunk_tokens(M, topk, N1, K1, N2, K2):
                 self.apply(output[t0:t1], hidden_states[t0:t1], w1, w2, topk_weights[t0:t1], topk_ids[t0:t1],
                            activation, global_num_experts, expert_map, a1q_scale, a2_scale, workspace13, workspace2,
                            expert_tokens_meta, apply_router_weight_on_input)
@@ -300,8 +309,8 @@ class R9700Mxfp4Experts(_experts_base()):
                 and MT == 1 and pf_gate is None and pf_down is None and K.stream_wanted(numel, E, topk)
                 and not K.down_sum_fits(numel, N2, K2)):
             W1, W2, (sid, eid, ntpp), _ = passes[0]
-            down = torch.empty((numel, N2), dtype=torch.bfloat16, device=dev)
-            tw = topk_weights.reshape(-1).to(torch.float32).contiguous()
+            down = K._empty(hidden_states, torch.bfloat16, numel, N2)
+            tw = _flat(topk_weights, torch.float32)
             if K.moe_stream_layer(xq, xs, W1, W2, down, sid, eid, ntpp, numel, topk, tw, E):
                 K.moe_sum(down.view(M, topk, N2), None, output)
                 return output
@@ -311,7 +320,7 @@ class R9700Mxfp4Experts(_experts_base()):
                 K.moe_gemm(xq, xs, W1, aq, sid, eid, ntpp, numel, topk, None, num_experts=E, MT=1, fuse=1)
             as_ = None
         else:
-            gate_up = torch.empty((numel, N1), dtype=torch.bfloat16, device=dev)
+            gate_up = K._empty(hidden_states, torch.bfloat16, numel, N1)
             for W1, _, (sid, eid, ntpp), (mt, pfg, _) in passes:
                 if mt == STREAM_PASS:
                     _stream_pass(xq, xs, W1, gate_up, sid, eid, ntpp, numel, topk, None, E)
@@ -320,11 +329,12 @@ class R9700Mxfp4Experts(_experts_base()):
                                prefill=pfg)
             # the token-major tail's expert ids: the routing ids, or each row's slot when every routed expert is
             # resident (the cache's one-launch manage wrote them; the host pass is provably empty)
-            ds_ids = topk_ids.to(torch.int32).contiguous() if cache is None else slot_ids
+            ds_ids = (topk_ids if topk_ids.dtype == torch.int32 and topk_ids.is_contiguous()
+                      else topk_ids.to(torch.int32).contiguous()) if cache is None else slot_ids
             if (ds_ids is not None and len(passes) == 1 and nv is None and expert_map is None and MT == 1
                     and pf_gate is None and K.down_sum_fits(numel, N2, K2) and not ZERO_DOWN):
                 # decode widths: SiLU + quant, down and the top-k sum in one token-major launch
-                tw = topk_weights.reshape(-1).to(torch.float32).contiguous()
+                tw = _flat(topk_weights, torch.float32)
                 if K.moe_down_sum(gate_up, ds_ids, tw, passes[0][1], output):
                     return output
             aq, as_ = K.silu_mul_quant_fp8(gate_up)
@@ -332,8 +342,8 @@ class R9700Mxfp4Experts(_experts_base()):
         if expert_map is not None or ZERO_DOWN:
             down = torch.zeros((numel, N2), dtype=torch.bfloat16, device=dev)
         else:
-            down = torch.empty((numel, N2), dtype=torch.bfloat16, device=dev)
-        tw = topk_weights.reshape(-1).to(torch.float32).contiguous()
+            down = K._empty(hidden_states, torch.bfloat16, numel, N2)
+        tw = _flat(topk_weights, torch.float32)
         for _, W2, (sid, eid, ntpp), (mt, _, pfd) in passes:
             if mt == STREAM_PASS:
                 _stream_pass(aq, as_, W2, down, sid, eid, ntpp, numel, 1, tw, E)

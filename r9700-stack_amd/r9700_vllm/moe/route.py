@@ -32,6 +32,7 @@ MAX_ROWS = int(os.environ.get("R9K_MOE_ROUTE_MAX_ROWS", "256"))
 QUANT_MAX_NUMEL = 4096              # routed rows (M * topk) r9k_moe_route_quant and _dual take in one launch
 _LIB = torch.library.Library("r9700", "FRAGMENT")
 _bound = None
+_limits: list = []                  # most experts and top-k the routing kernels take, once bound
 _registered = False
 
 
@@ -51,6 +52,7 @@ def lib() -> ctypes.CDLL:
         L.r9k_moe_route_dual.restype = i
         L.r9k_moe_route_max_experts.restype = i
         L.r9k_moe_route_max_topk.restype = i
+        _limits[:] = L.r9k_moe_route_max_experts(), L.r9k_moe_route_max_topk()
         _bound = L
     return _bound
 
@@ -78,18 +80,16 @@ def scratch_ints(E: int) -> int:
 def _launch(quant_x, logits, topk, renorm, blk, sorted_ids, expert_ids, ntpp, scratch):
     """One routing launch; with quant_x also the fp8 quant of that input. Returns (rc, w, ids, xq, xs)."""
     M, E = logits.shape
-    dev = logits.device
-    w = torch.empty((M, topk), dtype=torch.float32, device=dev)
-    ids = torch.empty((M, topk), dtype=torch.int32, device=dev)
-    head = (logits.data_ptr(), logits.stride(0), w.data_ptr(), ids.data_ptr(), sorted_ids.data_ptr(),
-            expert_ids.data_ptr(), ntpp.data_ptr(), scratch.data_ptr(), M, E, topk, int(bool(renorm)), blk)
-    st = torch.cuda.current_stream().cuda_stream
+    w = KM._empty(logits, torch.float32, M, topk)
+    ids = KM._empty(logits, torch.int32, M, topk)
+    head = (logits, logits.stride(0), w, ids, sorted_ids, expert_ids, ntpp, scratch, M, E, topk, int(bool(renorm)), blk)
+    st = KM._stream()
     if quant_x is None:
-        return lib().r9k_moe_route(*head, st), w, ids, None, None
+        return KM._call("r9k_moe_route", *head, st), w, ids, None, None
     H = quant_x.shape[1]
-    xq = torch.empty((M, H), dtype=torch.float8_e4m3fn, device=dev)
-    xs = torch.empty((M,), dtype=torch.float32, device=dev)
-    rc = lib().r9k_moe_route_quant(*head, quant_x.data_ptr(), quant_x.stride(0), H, xq.data_ptr(), xs.data_ptr(), st)
+    xq = KM._empty(logits, torch.float8_e4m3fn, M, H)
+    xs = KM._empty(logits, torch.float32, M)
+    rc = KM._call("r9k_moe_route_quant", *head, quant_x, quant_x.stride(0), H, xq, xs, st)
     return rc, w, ids, xq, xs
 
 
@@ -137,19 +137,16 @@ def moe_route_dual(logits: torch.Tensor, topk: int, renorm: bool, blk: int, sort
     ids = torch.empty((M, topk), dtype=torch.int32, device=dev)
     xq = torch.empty((0,), dtype=torch.float8_e4m3fn, device=dev)
     xs = torch.empty((0,), dtype=torch.float32, device=dev)
-    xa = (0, 0, 0, 0, 0)
+    xa = (None, 0, 0, None, None)
     if x is not None:
         if not (x.dim() == 2 and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.shape[0] == M):
             raise ValueError("moe_route_dual: x must be bf16 [M, H] with unit column stride")
         H = x.shape[1]
         xq = torch.empty((M, H), dtype=torch.float8_e4m3fn, device=dev)
         xs = torch.empty((M,), dtype=torch.float32, device=dev)
-        xa = (x.data_ptr(), x.stride(0), H, xq.data_ptr(), xs.data_ptr())
-    rc = lib().r9k_moe_route_dual(logits.data_ptr(), logits.stride(0), w.data_ptr(), ids.data_ptr(),
-                                  sorted_ids.data_ptr(), expert_ids.data_ptr(), ntpp.data_ptr(), scratch.data_ptr(),
-                                  M, E, topk, int(renorm), blk, *xa, big_blk, sorted_big.data_ptr(),
-                                  expert_big.data_ptr(), ntpp_big.data_ptr(), min_rows,
-                                  torch.cuda.current_stream().cuda_stream)
+        xa = (x, x.stride(0), H, xq, xs)
+    rc = KM._call("r9k_moe_route_dual", logits, logits.stride(0), w, ids, sorted_ids, expert_ids, ntpp, scratch, M, E,
+                  topk, int(renorm), blk, *xa, big_blk, sorted_big, expert_big, ntpp_big, min_rows, KM._stream())
     if rc:
         raise RuntimeError(f"r9k_moe_route_dual failed ({rc}) M={M} E={E} topk={topk} blk={blk} big={big_blk}")
     return w, ids, xq, xs
@@ -293,10 +290,10 @@ def plan_route(logits: torch.Tensor, topk: int, E: int, x, indices_type=None) ->
     """'decode', 'wide' or 'stock' for one router call (see the module docstring)."""
     if indices_type not in (None, torch.int32):
         return "stock"
-    L = lib()
+    if _bound is None:
+        lib()
     if not (logits.dim() == 2 and logits.dtype == torch.bfloat16 and logits.stride(1) == 1
-            and logits.shape[1] == E and E <= L.r9k_moe_route_max_experts()
-            and 1 <= topk <= min(E, L.r9k_moe_route_max_topk())):
+            and logits.shape[1] == E and E <= _limits[0] and 1 <= topk <= min(E, _limits[1])):
         return "stock"
     M = logits.shape[0]
     if 1 <= M <= MAX_ROWS:

@@ -24,7 +24,7 @@ import torch
 
 from .._compat import get_logger, register_custom_op
 from ..kernels import moe as KM
-from ..ops import _LIB, mxfp4_gemm_q
+from ..ops import _LIB, mxfp4_gemm_rows
 
 # the module classes whose gated shared expert the reference's model code hands to install (matched by name: vLLM's
 # classes are not importable without vLLM)
@@ -66,14 +66,14 @@ class SharedExpertWeights:
         """x [M, K1] bf16 contiguous -> [M, N2] bf16."""
         M = x.shape[0]
         W1, W2 = self.gate_up, self.down
-        y = torch.empty((M, W2.N), dtype=torch.bfloat16, device=x.device)
+        y = KM._empty(x, torch.bfloat16, M, W2.N)
         if M == 0:
             return y
         q, s, gate = KM.quant_rows_fp8_gate(x, self.wg)
-        h = torch.empty((M, W1.N), dtype=torch.bfloat16, device=x.device)
-        mxfp4_gemm_q(q, s, W1, h, M, KM.pick_cfg(W1.N, W1.K, M=M, kind="mxfp4", fold=W1.fold))
+        h = KM._empty(x, torch.bfloat16, M, W1.N)
+        mxfp4_gemm_rows(q, s, W1, h, M, W1.fold)
         hq, hs = KM.silu_mul_quant_fp8(h)
-        mxfp4_gemm_q(hq, hs, W2, y, M, KM.pick_cfg(W2.N, W2.K, M=M, kind="mxfp4", fold=W2.fold), topk_w=gate)
+        mxfp4_gemm_rows(hq, hs, W2, y, M, W2.fold, topk_w=gate)
         return y
 
 

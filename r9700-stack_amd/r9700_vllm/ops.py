@@ -16,6 +16,7 @@ from __future__ import annotations
 import torch
 
 from ._compat import register_custom_op
+from .kernels import moe as KM
 
 _LIB = torch.library.Library("r9700", "FRAGMENT")
 _registered = False
@@ -42,7 +43,6 @@ class IdentityTables:
 
 def _decode_mt(M: int) -> int:
     """M-tiles per routing block of a dense decode GEMM (kernels.moe.decode_mt)."""
-    from .kernels import moe as KM
     return KM.decode_mt(M)
 
 
@@ -50,7 +50,6 @@ def mxfp4_gemm_q(q: torch.Tensor, s: torch.Tensor, W, out: torch.Tensor, M: int,
     """out [M, W.N] bf16 = dequant(q, s) @ W^T (* topk_w[row]) for one dense MXFP4 weight, on the kernel `cfg` names:
     ("P", prefill cfg) or a decode tuple (WV, SK, NPW[, MT]) whose only meaning here is the optional MT. A decode cfg
     with at most KM.DENSE_A8_MAX_M rows runs on the dense kernel (r9k_dense_mxfp4_a8), the decode GEMM's bits."""
-    from .kernels import moe as KM
     if (not KM.is_prefill_cfg(cfg) and M <= KM.DENSE_A8_MAX_M and not W.fold
             and KM.dense_mxfp4_a8(q, s, W, out, topk_w)):
         return
@@ -61,6 +60,14 @@ def mxfp4_gemm_q(q: torch.Tensor, s: torch.Tensor, W, out: torch.Tensor, M: int,
     MT = cfg[3] if len(cfg) > 3 else _decode_mt(M)
     tabs = IdentityTables.get(q.device, M, KM.MOE_BLOCK * MT)
     KM.moe_gemm(q, s, W, out, *tabs, M, 1, topk_w, *cfg[:3], num_experts=1, MT=MT)
+
+
+def mxfp4_gemm_rows(q: torch.Tensor, s: torch.Tensor, W, out: torch.Tensor, M: int, fold: bool = False,
+                    topk_w=None) -> None:
+    """mxfp4_gemm_q on pick_cfg's choice (which the rows the dense kernel serves do without)."""
+    if M <= KM.DENSE_A8_MAX_M and not W.fold and KM.dense_mxfp4_a8(q, s, W, out, topk_w):
+        return
+    mxfp4_gemm_q(q, s, W, out, M, KM.pick_cfg(W.N, W.K, M=M, kind="mxfp4", fold=fold), topk_w=topk_w)
 
 
 # The prefill GEMMs address their activation rows and their output through 32-bit buffer ranges, so one launch may
@@ -79,29 +86,31 @@ def row_ranges(M: int, N: int, K: int, limit: int = BUF_LIMIT) -> list:
 
 
 def _mxfp4_linear_rows(x: torch.Tensor, W, out: torch.Tensor, fold: bool) -> None:
-    from .kernels import moe as KM
     M = x.shape[0]
     if M <= KM.DENSE_QA_MAX_M and not fold and KM.dense_mxfp4_qa(x, W, out):   # decode widths: quant in the launch
         return
     q, s = KM.quant_rows_fp8(x)
-    cfg = ("P", KM.MID_CFG) if M < KM.PREFILL_MIN_M and KM.dense_mid_wanted(M, W.N, W.K) else (
-        KM.pick_cfg(W.N, W.K, M=M, kind="mxfp4", fold=fold))
-    mxfp4_gemm_q(q, s, W, out, M, cfg)
+    if M < KM.PREFILL_MIN_M and KM.dense_mid_wanted(M, W.N, W.K):
+        mxfp4_gemm_q(q, s, W, out, M, ("P", KM.MID_CFG))
+    else:
+        mxfp4_gemm_rows(q, s, W, out, M, fold)
 
 
 def _mxfp4_linear(x: torch.Tensor, wq: torch.Tensor, wsr: torch.Tensor, N: int, K: int, fold: bool = False
                   ) -> torch.Tensor:
-    from .kernels import moe as KM
     M = x.shape[0]
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    out = KM._empty(x, torch.bfloat16, M, N)
     W = KM.Mxfp4Experts(wq, wsr, N, K, fold)
-    for r0, r1 in row_ranges(M, N, K):
+    ranges = row_ranges(M, N, K)
+    if len(ranges) == 1:
+        _mxfp4_linear_rows(x, W, out, fold)
+        return out
+    for r0, r1 in ranges:
         _mxfp4_linear_rows(x[r0:r1], W, out[r0:r1], fold)
     return out
 
 
 def _nvfp4_linear_rows(x: torch.Tensor, W, out: torch.Tensor) -> None:
-    from .kernels import moe as KM
     M = x.shape[0]
     if M <= KM.DENSE_NV_QA_MAX_M and KM.dense_nvfp4_qa(x, W, out):   # decode widths: the quant inside the GEMM launch
         return
@@ -120,11 +129,14 @@ def _nvfp4_linear(x: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, wg: torch
     """Native NVFP4 weights (prepare_nvfp4_weights of one expert) with per-row fp8 activations: one launch with the
     quant inside up to DENSE_NV_QA_MAX_M rows, the decode-family kernel below NV_PREFILL_MIN_M rows, the 128 x 128-tile
     prefill kernel (r9k_moe_4bit_prefill nv = 1) from there; row ranges past the 2 GiB buffer range (row_ranges)."""
-    from .kernels import moe as KM
     M = x.shape[0]
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    out = KM._empty(x, torch.bfloat16, M, N)
     W = KM.Nvfp4Experts(wq, ws, wg, N, K)
-    for r0, r1 in row_ranges(M, N, K):
+    ranges = row_ranges(M, N, K)
+    if len(ranges) == 1:
+        _nvfp4_linear_rows(x, W, out)
+        return out
+    for r0, r1 in ranges:
         _nvfp4_linear_rows(x[r0:r1], W, out[r0:r1])
     return out
 
@@ -157,10 +169,12 @@ def register() -> None:
 def _call_on_rows(op, x: torch.Tensor, K: int, N: int) -> torch.Tensor:
     """op over x viewed as contiguous bf16 rows [-1, K], the result shaped back to x's leading dims + [N]."""
     register()
-    rows = x.reshape(-1, K)
+    flat = x.dim() == 2 and x.shape[1] == K                    # rows already: no view to make and undo
+    rows = x if flat else x.reshape(-1, K)
     if rows.dtype != torch.bfloat16:
         rows = rows.to(torch.bfloat16)
-    return op(rows.contiguous()).reshape(*x.shape[:-1], N)
+    y = op(rows.contiguous())
+    return y if flat else y.reshape(*x.shape[:-1], N)
 
 
 def mxfp4_linear(x: torch.Tensor, wq: torch.Tensor, wsr: torch.Tensor, N: int, K: int, fold: bool = False

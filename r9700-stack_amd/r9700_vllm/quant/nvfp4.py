@@ -26,6 +26,7 @@ import os
 
 import torch
 
+from .. import ops
 from .._compat import get_logger
 from ..kernels import moe as KM
 
@@ -87,8 +88,7 @@ def nvfp4_to_mxfp4(packed, scale16, row_div, rows_per_chunk: int = 2048):
         d = row_div[r0:r1].to(dev, torch.float32).contiguous()
         dst_p = out_p[r0:r1] if on_gpu else torch.empty_like(p)
         dst_e = out_e[r0:r1] if on_gpu else torch.empty((r1 - r0, K // 32), dtype=torch.uint8, device=dev)
-        rc = KM.lib().r9k_nvfp4_to_mxfp4(p.data_ptr(), s.data_ptr(), d.data_ptr(), dst_p.data_ptr(),
-                                         dst_e.data_ptr(), r1 - r0, K, KM._stream())
+        rc = KM._call("r9k_nvfp4_to_mxfp4", p, s, d, dst_p, dst_e, r1 - r0, K, KM._stream())
         if rc:
             raise RuntimeError(f"r9k_nvfp4_to_mxfp4 failed ({rc}) rows={r1 - r0} K={K}")
         if not on_gpu:
@@ -147,7 +147,6 @@ def prepare_native_dense_layer(layer) -> None:
 
 
 def native_dense_forward(layer, x: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-    from .. import ops
     N, K = layer._r9k_nk
     y = ops.nvfp4_linear(x, layer.weight, layer.weight_scale, layer.weight_row_mult, N, K).to(x.dtype)
     return y if bias is None else y + bias
