@@ -255,7 +255,7 @@ struct NvPick { int NPW, SK, U; };
 // Launch shape from the host-known shape: two column tiles a workgroup (one for a dense linear of up to 8 rows); K
 // split over SK waves for long K; each wave issues its K range in as few load batches as 4 K-tiles a batch allow (5
 // for a dense linear of more than 8 rows).
-NvPick nv_pick(int N, int K, int max_blocks, int rows) {
+NvPick nv_pick(int N, int K, int max_blocks, int rows, int MT) {
   const int nkt = (K + NV_KT - 1) / NV_KT;
   const int NT = N / 16;
   const int NPW = NT >= 2 ? 2 : 1;
@@ -264,8 +264,8 @@ NvPick nv_pick(int N, int K, int max_blocks, int rows) {
   const int per = (nkt + SK - 1) / SK;
   int U = per >= 4 ? 4 : (per >= 2 ? 2 : 1);
   int npw = NPW;
-  if (max_blocks <= 2 && SK == 4 && per >= 5) {
-    // at most two routing blocks (a dense linear at decode widths: moe_gemm sizes the grid at ceil(numel / 16) +
+  if (MT == 1 && max_blocks <= 2 && SK == 4 && per >= 5) {
+    // at most two 16-row routing blocks (a dense linear at decode widths: moe_gemm sizes the grid at ceil(numel / 16) +
     // min(numel, E) blocks): one column tile a workgroup up to 8 rows, two and 5-tile
     // batches above (config 4, [17408, 5120], quant + GEMM: M = 1 19.6 -> 18.4 us, M = 4 19.5 -> 18.8, M = 16
     // 23.6 -> 22.8; the K split is unchanged, so the bits are too)
@@ -595,7 +595,7 @@ extern "C" int r9k_moe_nvfp4a8(long a, long as, long wq, long ws, long wg, long 
   if (max_blocks <= 0 || numel <= 0) return 0;
   if (!a || !as || !wq || !ws || !wg || !c || !sorted_ids || !expert_ids || !ntpp) return -3;
   const int blk = 16 * MT;
-  const NvPick p = nv_pick(N, K, max_blocks, numel);
+  const NvPick p = nv_pick(N, K, max_blocks, numel, MT);
   const dim3 grid((N / 16 + p.NPW - 1) / p.NPW, (unsigned)max_blocks);
   const long wq_estride = (long)N * ((K + NV_KT - 1) / NV_KT) * 64;
   const hipStream_t st = (hipStream_t)stream;
@@ -625,7 +625,7 @@ extern "C" int r9k_dense_nvfp4_qa(long x, long ldx, long wq, long ws, long wg, l
   if (M <= 0) return 0;
   if (!x || !wq || !ws || !wg || !out || N <= 0 || K <= 0) return -3;
   if (M > 2 || K % NV_KT || K > 8192 || N % 16 || (x & 15) || (ldx & 7) || (wq & 15)) return 2;
-  const NvPick p = nv_pick(N, K, 1, M);
+  const NvPick p = nv_pick(N, K, 1, M, 1);
   if (p.SK != 1 && p.SK != 4) return 2;
   const int T = WAVE * p.SK;
   if (K / 8 > (p.SK == 4 ? row_chunks<256>() : row_chunks<64>()) * T) return 2;

@@ -109,6 +109,12 @@ def test_nvfp4_linear(dev, M, N, Kd):
     check(O.bf16_bits(out), ref)
 
 
+@pytest.mark.parametrize("M", [31, 32, 33, 64, 65, 127])
+def test_nvfp4_linear_wide_decode_blocks(dev, M):
+    """Long K (5 K-tiles and more a wave) at 32- and 64-row routing blocks, where at most two blocks are launched."""
+    test_nvfp4_linear(dev, M, 144, 2560)
+
+
 @pytest.mark.parametrize("M,N,Kd", [(1, 17408, 5120), (2, 17408, 5120), (1, 1024, 2048), (2, 48, 1024),
                                     (1, 272, 384), (2, 64, 8192), (1, 16, 896), (2, 2064, 640)])
 def test_dense_nvfp4_qa_equals_two_launches(dev, M, N, Kd):
