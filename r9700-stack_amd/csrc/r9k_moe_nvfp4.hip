@@ -8,13 +8,13 @@
 // weight, exact, accumulated in fp32. Reference: kernels/r9k_moe_mxfp4a8.hip:89-96 and 300-340 (NVFP4 weight math),
 // :469-482 (epilogue order), :641-647 (entry).
 //
-// The scaled MFMA applies only power-of-two (e8m0) block scales, and the fp4 -> fp16 / bf16 conversions apply only
-// the exponent of their scale operand (both measured on gfx950), so an e4m3 scale rides on neither alone. Here each
-// group's scale s16 = 2^E * m (m in [1, 2), the e4m3 mantissa) is applied in two exact steps while the weights are
-// widened: V_CVT_SCALEF32_PK_F16_FP4 with s16 as its scale gives e2m1 * 2^E, and one packed fp16 multiply by m gives
-// e2m1 * s16 (at most 6 significant bits and within [2^-10, 2688]: exact in fp16). The fp8 activations widen to fp16
-// exactly (V_CVT_SCALEF32_PK_F16_FP8, scale 1), and V_MFMA_F32_16X16X32_F16 accumulates the exact products in fp32
-// -- no per-group rescaling of partial sums. A zero scale takes conversion scale 1 and m = 0.
+// The scaled MFMA applies only power-of-two (e8m0) block scales, so an e4m3 scale does not ride on it. Here the weights
+// are widened to fp16: V_CVT_SCALEF32_PK_F16_FP4 (scale 1) gives e2m1, one V_CVT_SCALEF32_PK_F16_FP8 a lane's two group
+// scales, and one packed fp16 multiply e2m1 * s16 (at most 6 significant bits and within [2^-10, 2688]: exact in fp16).
+// The fp8 activations widen to fp16 exactly, and V_MFMA_F32_16X16X32_F16 accumulates the exact products in fp32 -- no
+// per-group rescaling of partial sums. The widening's vector instructions bound these kernels next to the weight bytes
+// (decode) and the matrix pipe (prefill): splitting s16 into the conversion's exponent operand and a mantissa factor
+// took ~14 instructions a K-tile and column tile where this takes one.
 // Operand layout of the instruction: A lane l holds row l % 16 and 8 K values, B lane l column l % 16 and the same 8
 // K values, lane group g = l / 16 taking instruction K 8g .. 8g + 7; C lane l holds column l % 16, rows 4g .. 4g + 3.
 // Step s (0..3) of a 128-wide K-tile gives lane group g the K values 32g + 8s .. + 7, so over the tile lane group g
@@ -50,26 +50,18 @@ __device__ __forceinline__ uint32_t ld2_nt(const uint8_t* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const uint16_t*>(p));
 }
 
-// The two ways one e4m3 group scale enters the widening: the conversion scale (only its exponent is used) and the
-// packed fp16 mantissa factor.
-struct GroupScale {
-  float cvt;
-  h2 m;
-};
-__device__ __forceinline__ GroupScale group_scale(uint32_t byte) {
-  const float sf = __builtin_amdgcn_cvt_f32_fp8((int)byte, 0);
-  const float m = __uint_as_float((__float_as_uint(sf) & 0x807fffffu) | 0x3f800000u);
-  const bool z = sf == 0.f;
-  const float mz = z ? 0.f : m;
-  return {z ? 1.f : sf, (h2){(_Float16)mz, (_Float16)mz}};
+// The two e4m3 group scales of a lane's K-tile (the low 16 bits of sw) as fp16, exact; NaN bytes stay NaN.
+__device__ __forceinline__ h2 scales_f16(uint32_t sw) {
+  return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)sw, 1.0f, false);
 }
 
-// 8 e2m1 codes (one dword, low nibble first) -> e2m1 * s16 as 8 fp16, exact
-__device__ __forceinline__ h8 e2m1x8_f16(uint32_t w, GroupScale gs) {
-  const h2 p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, gs.cvt, 0) * gs.m;
-  const h2 p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, gs.cvt, 1) * gs.m;
-  const h2 p2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, gs.cvt, 2) * gs.m;
-  const h2 p3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, gs.cvt, 3) * gs.m;
+// 8 e2m1 codes (one dword, low nibble first) -> e2m1 * s as 8 fp16, exact
+__device__ __forceinline__ h8 e2m1x8_f16(uint32_t w, _Float16 s) {
+  const h2 ss = {s, s};
+  const h2 p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0) * ss;
+  const h2 p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1) * ss;
+  const h2 p2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2) * ss;
+  const h2 p3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3) * ss;
   return (h8){p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
 
@@ -181,10 +173,10 @@ __global__ void __launch_bounds__(WAVE * SK) moe_nvfp4_kernel(
         }
 #pragma unroll
         for (int j = 0; j < NPW; j++) {
-          const GroupScale s0 = group_scale(sw[u][j] & 0xffu), s1 = group_scale((sw[u][j] >> 8) & 0xffu);
+          const h2 gs = scales_f16(sw[u][j]);
 #pragma unroll
           for (int st = 0; st < 4; st++) {
-            const h8 b = e2m1x8_f16(bw[u][j][st], st < 2 ? s0 : s1);
+            const h8 b = e2m1x8_f16(bw[u][j][st], gs[st >> 1]);
 #pragma unroll
             for (int i = 0; i < MT; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][st], b, acc[j][i], 0, 0, 0);
           }
@@ -394,9 +386,9 @@ __global__ void __launch_bounds__(PV_THREADS, 2) nvfp4_prefill_kernel(
       const int ntl = wn * 4 + j;
       const u32x4 bw = *reinterpret_cast<const u32x4*>(S.b + ntl * 1024 + lane * 16);
       const uint32_t sw = *reinterpret_cast<const uint16_t*>(S.s + ntl * 128 + lane * 2);
-      const GroupScale s0 = group_scale(sw & 0xffu), s1 = group_scale((sw >> 8) & 0xffu);
+      const h2 gs = scales_f16(sw);
 #pragma unroll
-      for (int t = 0; t < 4; t++) b[j][t] = e2m1x8_f16(bw[t], t < 2 ? s0 : s1);
+      for (int t = 0; t < 4; t++) b[j][t] = e2m1x8_f16(bw[t], gs[t >> 1]);
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -516,10 +508,10 @@ __global__ void __launch_bounds__(WAVE * SK) dense_nvfp4_qa_kernel(
         const h8 a[4] = {e4m3x8_f16(l.x, l.y), e4m3x8_f16(l.z, l.w), e4m3x8_f16(h.x, h.y), e4m3x8_f16(h.z, h.w)};
 #pragma unroll
         for (int j = 0; j < NPW; j++) {
-          const GroupScale s0 = group_scale(sw[u][j] & 0xffu), s1 = group_scale((sw[u][j] >> 8) & 0xffu);
+          const h2 gs = scales_f16(sw[u][j]);
 #pragma unroll
           for (int st = 0; st < 4; st++) {
-            const h8 b = e2m1x8_f16(bw[u][j][st], st < 2 ? s0 : s1);
+            const h8 b = e2m1x8_f16(bw[u][j][st], gs[st >> 1]);
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[st], b, acc[j], 0, 0, 0);
           }
         }
