@@ -541,6 +541,76 @@ __global__ void __launch_bounds__(WAVE * SK) dense_nvfp4_qa_kernel(
   }
 }
 
+// ------------------------------------------------------------------- dense linear at decode widths, codes given
+// The native NVFP4 dense linear for M <= 16 rows already quantised: moe_nvfp4_kernel's weight stream for one routing
+// block of identity rows without the tables -- the same widening, MFMA order, K split over SK waves and partial-tile
+// sum, so the same bits. Bound by the weight bytes and the widening's issue slots. Against that kernel over identity
+// tables it starts its weight loads with its first instructions (no ntpp -> expert -> row id chain before them),
+// launches no workgroups for a second, empty block, and refills a K-tile's registers as soon as the tile is widened
+// instead of draining a batch before the next. One column tile a workgroup and two K-tiles in flight a wave: 80
+// registers, six waves a SIMD, which hide more than a deeper ring on fewer waves (MI355X, GEMM alone, [17408, 5120] at
+// M = 4: 14.2 us; 3 tiles 15.2, 4 15.2, 5 15.5, 10 16.1). Decode kernel -> this one, us: [17408, 5120] M = 4 / 8 / 16
+// 16.1 / 17.9 / 20.3 -> 14.2 / 15.0 / 18.3, [5120, 17408] 22.4 / 23.5 / 27.0 -> 19.2 / 18.9 / 21.9, [4096, 4096]
+// 7.3 / 7.5 / 10.4 -> 6.6 / 6.5 / 7.0, [1024, 2048] 6.0 / 6.1 / 6.5 -> 4.6 / 4.7 / 4.9.
+template <int SK>
+__global__ void __launch_bounds__(WAVE * SK) dense_nvfp4_a8_kernel(
+    const uint8_t* __restrict__ A, long lda, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
+    const uint8_t* __restrict__ Ws, const float* __restrict__ Wg, uint16_t* __restrict__ out, long ldo, int M, int K) {
+  constexpr int U = 2;                                          // K-tiles in flight a wave
+  __shared__ float red[SK * 256];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  const int g = lane >> 4, c = lane & 15;
+  const int nt = blockIdx.x, nkt = K / NV_KT;
+  const uint8_t* wtile = Wq + (size_t)nt * nkt * 1024 + lane * 16;
+  const uint8_t* stile = Ws + (size_t)nt * nkt * 128 + lane * 2;
+  const uint8_t* arow = A + (size_t)min(c, M - 1) * lda + 32 * g;   // rows past M compute a copy, never stored
+  const int kt0 = wave * nkt / SK, kt1 = (wave + 1) * nkt / SK;
+
+  u32x4 bw[U];
+  uint32_t sw[U];
+  uint4 lo[U], hi[U];
+  auto issue = [&](int u, int k) {
+    bw[u] = ld16_nt(wtile + (size_t)k * 1024);
+    sw[u] = ld2_nt(stile + (size_t)k * 128);
+    lo[u] = *reinterpret_cast<const uint4*>(arow + (size_t)k * NV_KT);
+    hi[u] = *reinterpret_cast<const uint4*>(arow + (size_t)k * NV_KT + 16);
+  };
+#pragma unroll
+  for (int u = 0; u < U; u++) issue(u, min(kt0 + u, nkt - 1));
+  // this thread's outputs: column tid % 16 of the tile, row tid / 16 and on
+  const int n = nt * 16 + (tid & 15);
+  const float wgn = Wg[n];
+
+  v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
+  for (int kt = kt0; kt < kt1; kt += U) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (kt + u < kt1) {                                    // wave-uniform
+        const h8 a[4] = {e4m3x8_f16(lo[u].x, lo[u].y), e4m3x8_f16(lo[u].z, lo[u].w), e4m3x8_f16(hi[u].x, hi[u].y),
+                         e4m3x8_f16(hi[u].z, hi[u].w)};
+        const h2 gs = scales_f16(sw[u]);
+        h8 b[4];
+#pragma unroll
+        for (int st = 0; st < 4; st++) b[st] = e2m1x8_f16(bw[u][st], gs[st >> 1]);
+        if (kt + u + U < kt1) issue(u, kt + u + U);
+#pragma unroll
+        for (int st = 0; st < 4; st++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[st], b[st], acc, 0, 0, 0);
+      }
+    }
+  }
+
+#pragma unroll
+  for (int q = 0; q < 4; q++) red[wave * 256 + (4 * g + q) * 16 + c] = acc[q];
+  __syncthreads();
+  for (int m = tid >> 4; m < M; m += WAVE * SK / 16) {
+    float v = 0.f;
+#pragma unroll
+    for (int s = 0; s < SK; s++) v += red[s * 256 + m * 16 + (tid & 15)];
+    const float sc = wgn * As[m];
+    out[(size_t)m * ldo + n] = f2bf(v * sc);
+  }
+}
+
 }  // namespace
 
 // The prefill entry's native-NVFP4 case (r9k_moe_4bit_prefill with nv = 1; reference kernels/r9k_moe_mxfp4a8.hip:
@@ -639,4 +709,27 @@ extern "C" int r9k_dense_nvfp4_qa(long x, long ldx, long wq, long ws, long wg, l
 #undef NQM
 #undef NQ
   return 2;
+}
+
+// No counterpart as one entry in the reference: the GEMM half of r9k_quant_rows_fp8 + r9k_moe_nvfp4a8 over identity
+// tables (the native NVFP4 dense linear, r9700_vllm/ops.py:66-83) for 1 <= M <= 16 pre-quantised rows. q fp8 [M][K]
+// (row stride ldq bytes, rows 16-byte aligned), s fp32 [M]; wq / ws / wg one expert in this kernel's layout; out bf16
+// [M][N] (row stride ldo). Served: 1 <= M <= 16, K % 128 == 0, N % 16 == 0; 2 (nothing launched) otherwise. 0, -3 bad
+// argument, -6 launch error. Same K split as r9k_moe_nvfp4a8 for one block, so the same bits.
+extern "C" int r9k_dense_nvfp4_a8(long q, long ldq, long s, long wq, long ws, long wg, long out, long ldo, int M,
+                                  int N, int K, long stream) {
+  if (M <= 0) return 0;
+  if (!q || !s || !wq || !ws || !wg || !out || N <= 0 || K <= 0) return -3;
+  if (M > 16 || K % NV_KT || N % 16 || (q & 15) || (ldq & 15) || (wq & 15) || (ws & 1)) return 2;
+  const int SK = nv_pick(N, K, 1, M, 1).SK;
+  const dim3 grid(N / 16), block(WAVE * SK);
+#define NA(SKv)                                                                                                     \
+  hipLaunchKernelGGL((dense_nvfp4_a8_kernel<SKv>), grid, block, 0, (hipStream_t)stream, (const uint8_t*)q, ldq,     \
+                     (const float*)s, (const uint8_t*)wq, (const uint8_t*)ws, (const float*)wg, (uint16_t*)out, ldo, \
+                     M, K)
+  if (SK == 1) NA(1);
+  else if (SK == 2) NA(2);
+  else NA(4);
+#undef NA
+  return hipGetLastError() == hipSuccess ? 0 : -6;
 }

@@ -84,6 +84,8 @@ def lib() -> ctypes.CDLL:
         L.r9k_dense_nvfp4_qa.restype = i
         L.r9k_dense_nvfp4_qa.argtypes = [l] * 7 + [i] * 3 + [l]
         L.r9k_dense_mxfp4_a8.argtypes = [l] * 8 + [i] * 3 + [l]
+        L.r9k_dense_nvfp4_a8.restype = i
+        L.r9k_dense_nvfp4_a8.argtypes = [l] * 8 + [i] * 3 + [l]
         L.r9k_moe_down_sum.argtypes = [l] * 10 + [i] * 5 + [l]
         L.r9k_moe_stream.restype = i
         L.r9k_moe_stream.argtypes = [i] + [l] * 11 + [i] * 6 + [l]
@@ -917,6 +919,28 @@ def dense_nvfp4_qa(x: torch.Tensor, w: Nvfp4Experts, out: torch.Tensor) -> bool:
         return False
     if rc:
         raise RuntimeError(f"r9k_dense_nvfp4_qa failed ({rc}) M={M} N={w.N} K={w.K}")
+    return True
+
+
+# ops.nvfp4_linear's GEMM on quantised rows runs the dense kernel (r9k_dense_nvfp4_a8) up to this many rows (all it
+# serves), above them the decode-family kernel over identity tables. Measured on MI355X, decode kernel -> dense kernel,
+# us: [17408, 5120] M = 4 / 16 16.1 / 20.3 -> 14.2 / 18.3, [1024, 2048] 6.0 / 6.5 -> 4.6 / 4.9.
+DENSE_NV_A8_MAX_M = int(os.environ.get("R9K_DENSE_NV_A8_MAX_M", "16"))
+
+
+def dense_nvfp4_a8(q: torch.Tensor, s: torch.Tensor, w: Nvfp4Experts, out: torch.Tensor) -> bool:
+    """out [M, N] = bf16(dequant(q, s) @ W^T) for one native NVFP4 weight and M <= 16 rows already quantised
+    (quant_rows_fp8's codes and scales), without routing tables (r9k_dense_nvfp4_a8): the values of moe_gemm over
+    identity tables bit for bit. False when not served (nothing launched)."""
+    M = q.shape[0]
+    assert q.dtype in (torch.uint8, torch.float8_e4m3fn) and q.dim() == 2 and q.stride(1) == 1 and q.shape[1] == w.K
+    assert s.dtype == torch.float32 and s.is_contiguous() and s.numel() >= M
+    assert out.dtype == torch.bfloat16 and out.shape == (M, w.N) and out.stride(1) == 1
+    rc = _call("r9k_dense_nvfp4_a8", q, q.stride(0), s, w.wq, w.ws, w.wg, out, out.stride(0), M, w.N, w.K, _stream())
+    if rc == 2:
+        return False
+    if rc:
+        raise RuntimeError(f"r9k_dense_nvfp4_a8 failed ({rc}) M={M} N={w.N} K={w.K}")
     return True
 
 

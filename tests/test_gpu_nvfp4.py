@@ -141,6 +141,35 @@ def test_dense_nvfp4_qa_equals_two_launches(dev, M, N, Kd):
     check(O.bf16_bits(one), ref)
 
 
+@pytest.mark.parametrize("M,N,Kd", [(1, 1024, 2048), (3, 48, 128), (4, 17408, 5120), (5, 272, 384), (8, 16, 896),
+                                    (9, 2064, 640), (15, 64, 8192), (16, 144, 1152)])
+def test_dense_nvfp4_a8_equals_decode_gemm(dev, M, N, Kd):
+    """r9k_dense_nvfp4_a8 (pre-quantised rows, no tables) against the decode kernel over identity tables: bit for bit,
+    every output written, rows of a wider buffer (strides) included; unserved widths launch nothing."""
+    print(f"dense nvfp4 a8 M={M} N={N} K={Kd}", flush=True)
+    g = torch.Generator().manual_seed(20261201 + 4400 + M + N + Kd)
+    packed, s16, wg = make_nv(1, N, Kd, g)
+    W = K.prepare_nvfp4_weights(packed.to(dev), s16.to(dev), wg.to(dev))
+    x = torch.randn(M, Kd, generator=g).to(torch.bfloat16)
+    q, s = K.quant_rows_fp8(x.to(dev))
+    wide = torch.zeros(M, Kd + 32, dtype=q.dtype, device=dev)
+    wide[:, :Kd] = q
+    buf = torch.full((M, N + 8), float("nan"), dtype=torch.bfloat16, device=dev)
+    assert K.dense_nvfp4_a8(wide[:, :Kd], s, W, buf[:, :N]), "shape not served"
+    two = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    K.moe_gemm(q, s, W, two, *ops.IdentityTables.get(dev, M, K.MOE_BLOCK), M, 1, None, num_experts=1, MT=1)
+    torch.cuda.synchronize()
+    assert torch.equal(buf[:, :N].contiguous().view(torch.int16), two.view(torch.int16))
+    assert torch.isnan(buf[:, N:].float()).all(), "columns past N were written"
+    wide17 = torch.zeros(17, Kd, dtype=q.dtype, device=dev)
+    assert not K.dense_nvfp4_a8(wide17, torch.ones(17, device=dev), W,
+                                torch.empty(17, N, dtype=torch.bfloat16, device=dev))
+    qo, so = O.quant_rows_fp8(x)
+    ref = O.nvfp4_gemm(qo, so, packed.numpy(), s16.view(torch.uint8).numpy(), wg.numpy(),
+                       np.zeros(M, dtype=np.int32), 1)
+    check(O.bf16_bits(buf[:, :N].contiguous()), ref)
+
+
 def test_dense_nvfp4_qa_refuses_unserved(dev):
     """M > 2 or K not a multiple of 128: False, nothing launched (ops falls back to the two launches)."""
     g = torch.Generator().manual_seed(7)
