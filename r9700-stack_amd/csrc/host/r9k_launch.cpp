@@ -70,7 +70,12 @@ PyObject* py_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       return nullptr;
     }
   }
-  return PyLong_FromLong(dispatch<1>((size_t)nargs - 1, fn, v));
+  // without the GIL, as ctypes calls it: a launch waits while its queue is full, and another thread may have to run first
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = dispatch<1>((size_t)nargs - 1, fn, v);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
 

@@ -209,14 +209,17 @@ def prepare_nvfp4_weights(packed: torch.Tensor, scale16: torch.Tensor, row_mult:
 
 def _prep_kernel(packed: torch.Tensor | None, scale: torch.Tensor | None, wq: torch.Tensor | None,
                  wsr: torch.Tensor | None) -> bool:
-    """permute_fragments and / or pack_scales in one launch (r9k_mxfp4_prep) for contiguous, aligned tensors on the
-    current GPU; False (nothing launched) for anything else: the torch expressions then do it."""
+    """permute_fragments and / or pack_scales in one launch (r9k_mxfp4_prep) for contiguous, aligned tensors of exactly
+    the kernel's sizes on the current GPU; False (nothing launched) for anything else: the torch expressions then do it,
+    or refuse it."""
     ts = [t for t in (packed, scale, wq, wsr) if t is not None]
     src = packed if packed is not None else scale
     E, N, cols = src.shape
     K = cols * (2 if packed is not None else GROUP)
     if not (all(t.is_cuda and t.is_contiguous() and t.device.index == torch.cuda.current_device() for t in ts)
             and N % 16 == 0 and K % GROUP == 0 and 0 < E <= 65535 and K > 0
+            and (packed is None or wq.numel() * wq.element_size() == packed.numel())
+            and (scale is None or wsr.shape == (E, K // GROUP + 1, N))
             and all(t.data_ptr() % 16 == 0 for t in (packed, wq) if t is not None)
             and (wsr is None or wsr.data_ptr() % 4 == 0)):
         return False

@@ -28,6 +28,20 @@ def test_prep_equals_torch(dev, E, N, Kd):
     assert off.data_ptr() % 16 and torch.equal(K.permute_fragments(off).cpu(), ref_q)
 
 
+def test_prep_output_sizes(dev):
+    """An `out` of another size never reaches the kernel: too small is refused, a longer scale tensor keeps its tail."""
+    E, N, Kd = 2, 32, 128
+    packed, e8 = make_experts(E, N, Kd, torch.Generator().manual_seed(5), lo=0, hi=255)
+    small = torch.empty(E * N * Kd // 2 - 16, dtype=torch.uint8, device=dev)
+    with pytest.raises(RuntimeError):
+        K.permute_fragments(packed.to(dev), out=small)
+    with pytest.raises((RuntimeError, IndexError)):
+        K.pack_scales(e8.to(dev), out=torch.empty((E, Kd // 32, N), dtype=torch.uint8, device=dev))
+    long = torch.full((E, Kd // 32 + 2, N), 7, dtype=torch.uint8, device=dev)
+    K.pack_scales(e8.to(dev), out=long)
+    assert torch.equal(long[:, :-1].cpu(), K.pack_scales(e8)) and bool((long[:, -1] == 7).all())
+
+
 @pytest.mark.parametrize("rd", [1.0, 448.0, 2688.0 / 3.7, 1e30, 1e-30, 3.3e38])
 def test_nvfp4_search_branches(dev, rd):
     """Uniform blocks, every scale byte (zero, subnormal, negative, NaN), one-magnitude and all-zero blocks, groups whose
