@@ -30,7 +30,7 @@ CFLAGS = [
 # Per-source additions. The prefill GEMM interleaves its MFMAs with LDS reads and DMA issue under scheduling
 # barriers; machine sinking would move the MFMAs (pure operations) past the loop's wait/barrier branches into one
 # block at the end of the loop body and undo that order.
-FILE_FLAGS = {f: ["-mllvm", "-disable-machine-sink"] for f in ("r9k_moe_prefill.hip", "r9k_moe_mid.hip")}
+FILE_FLAGS = {f: ["-mllvm", "-disable-machine-sink"] for f in ("r9k_moe_prefill.hip", "r9k_moe_mid.hip", "r9k_moe_nvfp4.hip")}
 
 
 def hipcc() -> str:

@@ -65,6 +65,14 @@ __device__ __forceinline__ h8 e2m1x8_f16(uint32_t w, _Float16 s) {
   return (h8){p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
 
+// the two e2m1 codes of byte j (constant) of one dword as fp16
+__device__ __forceinline__ h2 e2m1x2_f16(uint32_t w, int j) {
+  return j == 0 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0)
+       : j == 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1)
+       : j == 2 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2)
+                : __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3);
+}
+
 // 8 e4m3 codes (two dwords) -> 8 fp16, exact
 __device__ __forceinline__ h8 e4m3x8_f16(uint32_t lo, uint32_t hi) {
   const h2 p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)lo, 1.0f, false);
@@ -298,6 +306,7 @@ struct PvStage {
   uint8_t b[8 * 1024];             // codes of the 8 column tiles, the global layout's K-tile
   uint8_t s[8 * 128];              // their scales
 };
+struct PvW { u32x4 k[4]; };           // a column tile's widened weights of one K-tile
 constexpr size_t PV_SMEM = PV_NS * sizeof(PvStage) + PV_BM * (sizeof(int) + 2 * sizeof(float));
 
 __global__ void __launch_bounds__(PV_THREADS, 2) nvfp4_prefill_kernel(
@@ -353,15 +362,31 @@ __global__ void __launch_bounds__(PV_THREADS, 2) nvfp4_prefill_kernel(
   const uint32_t la0 = lds_addr(&st[0].a[wave * 1024]);
   const uint32_t lb0 = lds_addr(&st[0].b[wave * 1024]);
   const uint32_t ls0 = lds_addr(&st[0].s[wave * 256]);
-  auto issue = [&](int kt, int sg) {
-    const uint32_t so = (uint32_t)(sg * (int)sizeof(PvStage));
-    const uint32_t ka = (uint32_t)min(kt * NV_KT + gp16, K - 16);
+  // K-tile k's activations (4 loads) and codes + scales (3 loads) into ring slot sl; k past the end re-reads the last
+  // K-tile, so every step issues the same loads
+  auto issue_a = [&](int k, uint32_t sl) {
+    const uint32_t ka = (uint32_t)min(min(k, nkt - 1) * NV_KT + gp16, K - 16);
 #pragma unroll
-    for (int i = 0; i < 4; i++) dma16s(A, arow[i] + ka, la0 + so + i * 4096);
-#pragma unroll
-    for (int i = 0; i < 2; i++) dma16s(We, boff[i] + (uint32_t)kt * 1024u, lb0 + so + i * 4096);
-    dma4s(Se, soff + (uint32_t)kt * 128u, ls0 + so);
+    for (int i = 0; i < 4; i++) dma16s(A, arow[i] + ka, la0 + sl + i * 4096);
   };
+  auto issue_w = [&](int k, uint32_t sl) {
+    const uint32_t kc = (uint32_t)min(k, nkt - 1);
+#pragma unroll
+    for (int i = 0; i < 2; i++) dma16s(We, boff[i] + kc * 1024u, lb0 + sl + i * 4096);
+    dma4s(Se, soff + kc * 128u, ls0 + sl);
+  };
+
+  constexpr uint32_t SL = sizeof(PvStage);
+  // this lane's fragments in slot 0: row tile i at + i * 16 * NV_KT, column tile j at + j * 1024 (codes), + j * 128
+  const int r0 = wm * 64 + c;
+  const uint8_t* const fl = st[0].a + r0 * NV_KT + ((2 * g) ^ (r0 & 7)) * 16;
+  const uint8_t* const fh = st[0].a + r0 * NV_KT + ((2 * g + 1) ^ (r0 & 7)) * 16;
+  const uint8_t* const fw = st[0].b + wn * 4096 + lane * 16;
+  const uint8_t* const fs = st[0].s + wn * 512 + lane * 2;
+  auto ld_lo = [&](uint32_t sl, int i) { return *reinterpret_cast<const u32x4*>(fl + sl + i * 16 * NV_KT); };
+  auto ld_hi = [&](uint32_t sl, int i) { return *reinterpret_cast<const u32x4*>(fh + sl + i * 16 * NV_KT); };
+  auto ld_w = [&](uint32_t sl, int j) { return *reinterpret_cast<const u32x4*>(fw + sl + j * 1024); };
+  auto ld_s = [&](uint32_t sl, int j) { return (uint32_t)*reinterpret_cast<const uint16_t*>(fs + sl + j * 128); };
 
   v4f acc[4][4];
 #pragma unroll
@@ -369,44 +394,92 @@ __global__ void __launch_bounds__(PV_THREADS, 2) nvfp4_prefill_kernel(
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-  issue(0, 0);
-  if (nkt > 1) issue(1, 1);
-  int sidx = 0;
-  for (int kt = 0; kt < nkt; kt++) {
-    // K-tile kt is in once only the next one's DMA (when issued) is outstanding
-    if (kt + 1 < nkt) asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    // K-tile kt + 2 into the stage every wave finished reading in the previous iteration
-    if (kt + 2 < nkt) issue(kt + 2, sidx == 0 ? PV_NS - 1 : sidx - 1);
-    const PvStage& S = st[sidx];
-    h8 b[4][4];
+  // Ahead of the loop: K-tiles 0 and 1 of everything and 2 of the weights on their way, K-tile 0's weights widened, the
+  // raw weights of K-tile 1's first two column tiles and the raw activations of row tile 1 in registers
+  issue_a(0, 0);
+  issue_w(0, 0);
+  issue_w(1, SL);
+  issue_a(1, SL);
+  issue_w(2, 2 * SL);
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(PV_DMA) : "memory");
+  PvW B[2][3], b3;                                             // column tile 3 is widened in place
+  u32x4 a[4], rl = ld_lo(0, 0), rh = ld_hi(0, 0), rw[2];
+  uint32_t rs;
+  h2 gs;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int ntl = wn * 4 + j;
-      const u32x4 bw = *reinterpret_cast<const u32x4*>(S.b + ntl * 1024 + lane * 16);
-      const uint32_t sw = *reinterpret_cast<const uint16_t*>(S.s + ntl * 128 + lane * 2);
-      const h2 gs = scales_f16(sw);
+  for (int j = 0; j < 4; j++) {
+    rw[1] = ld_w(0, j);
+    gs = scales_f16(ld_s(0, j));
+    PvW& d = j < 3 ? B[0][j] : b3;
 #pragma unroll
-      for (int t = 0; t < 4; t++) b[j][t] = e2m1x8_f16(bw[t], gs[t >> 1]);
-    }
+    for (int t = 0; t < 4; t++) d.k[t] = __builtin_bit_cast(u32x4, e2m1x8_f16(rw[1][t], gs[t >> 1]));
+  }
+  a[0] = __builtin_bit_cast(u32x4, e4m3x8_f16(rl.x, rl.y));
+  a[1] = __builtin_bit_cast(u32x4, e4m3x8_f16(rl.z, rl.w));
+  a[2] = __builtin_bit_cast(u32x4, e4m3x8_f16(rh.x, rh.y));
+  a[3] = __builtin_bit_cast(u32x4, e4m3x8_f16(rh.z, rh.w));
+  rl = ld_lo(0, 1);
+  rw[0] = ld_w(SL, 0);
+  rs = ld_s(SL, 0);
+  __builtin_amdgcn_s_waitcnt(0xC07F);                          // K-tile 0's weights are read: slot 0 takes K-tile 3's
+  asm volatile("s_barrier" ::: "memory");
+  issue_a(2, 2 * SL);
+  issue_w(3, 0);
+
+  // One K-tile kt (slot c0; c1, c2 hold kt + 1, kt + 2) from the widened weights bc and b3. Row tile i's 16 MFMAs run
+  // step by step (p / 4) over the 4 column tiles, and each carries one conversion pair of row tile i + 1's activations
+  // and one of the next K-tile's column tile i, four MFMAs behind, so that activations and column tile 3 replace their
+  // predecessors in the same registers right after their last use (step 3 of each in the next row tile's first four).
+  // In row tile 2 a barrier publishes the activations of kt + 1 and the weights of kt + 2 (issued a K-tile ago; the 7
+  // loads after them stay in flight); every wave has read the activations of kt and the weights of kt + 1 by then, so
+  // their slots take those of kt + 3 and kt + 4.
+  auto step = [&](int kt, uint32_t c0, uint32_t c1, uint32_t c2, PvW (&bc)[3], PvW (&bn)[3]) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int r = (wm * 4 + i) * 16 + c;
-      const uint4 l = *reinterpret_cast<const uint4*>(S.a + r * NV_KT + (((2 * g) ^ (r & 7)) * 16));
-      const uint4 h = *reinterpret_cast<const uint4*>(S.a + r * NV_KT + (((2 * g + 1) ^ (r & 7)) * 16));
-      const h8 a0 = e4m3x8_f16(l.x, l.y), a1 = e4m3x8_f16(l.z, l.w), a2 = e4m3x8_f16(h.x, h.y),
-               a3 = e4m3x8_f16(h.z, h.w);
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b[j][0], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b[j][1], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a2, b[j][2], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a3, b[j][3], acc[i][j], 0, 0, 0);
+      for (int p = 0; p < 16; p++) {
+        if (i == 2 && p == 8) {
+          __builtin_amdgcn_s_waitcnt(0xC07F);
+          asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(PV_DMA) : "memory");
+          issue_a(kt + 3, c0);
+          issue_w(kt + 4, c1);
+        }
+        const int t = p >> 2, j = p & 3;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            __builtin_bit_cast(h8, a[t]), __builtin_bit_cast(h8, (j < 3 ? bc[j] : b3).k[t]), acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (p == 4) {
+          gs = scales_f16(rs);
+          rh = i < 3 ? ld_hi(c0, i + 1) : ld_hi(c1, 0);
+          rw[(i + 1) & 1] = i < 3 ? ld_w(c1, i + 1) : ld_w(c2, 0);
+          rs = i < 3 ? ld_s(c1, i + 1) : ld_s(c2, 0);
+        }
+        if (p == 12) rl = i < 2 ? ld_lo(c0, i + 2) : ld_lo(c1, i - 2);
+        const int u = p >= 4 ? t - 1 : 3;                      // the step converted here
+        const int jc = p >= 4 ? i : (i + 3) & 3;               // and its column tile (i == 0: of this K-tile)
+        const uint32_t av = u < 2 ? rl[2 * u + (j >> 1)] : rh[2 * u + (j >> 1) - 4];
+        const h2 pa = j & 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)av, 1.0f, true)
+                            : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)av, 1.0f, false);
+        a[u][j] = __builtin_bit_cast(uint32_t, pa);
+        const h2 pw = e2m1x2_f16(rw[jc & 1][u], j) * (h2){gs[u >> 1], gs[u >> 1]};
+        (jc < 3 ? bn[jc] : b3).k[u][j] = __builtin_bit_cast(uint32_t, pw);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    sidx = sidx == PV_NS - 1 ? 0 : sidx + 1;
+  };
+  uint32_t c0 = 0, c1 = SL, c2 = 2 * SL;
+  int kt = 0;
+  for (; kt + 1 < nkt; kt += 2) {
+    step(kt, c0, c1, c2, B[0], B[1]);
+    step(kt + 1, c1, c2, c0, B[1], B[0]);
+    const uint32_t x = c0;
+    c0 = c2;
+    c2 = c1;
+    c1 = x;
   }
+  if (kt < nkt) step(kt, c0, c1, c2, B[0], B[1]);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // no DMA may outlive the workgroup's LDS
 
   // epilogue: lane holds column c of each column tile, rows 4g .. 4g + 3 of each row tile; out = bf16(v * ((Wg[n] *
   // As[row]) * topk_w[row])), the row factors from LDS and the lane's 4 column multipliers loaded together. Branch-free:
