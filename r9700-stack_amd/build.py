@@ -27,10 +27,11 @@ CFLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",  # no packed fp32 VALU ops
     "-Wno-unused-command-line-argument",
 ]
-# Per-source additions. The prefill GEMM interleaves its MFMAs with LDS reads and DMA issue under scheduling
-# barriers; machine sinking would move the MFMAs (pure operations) past the loop's wait/barrier branches into one
-# block at the end of the loop body and undo that order.
-FILE_FLAGS = {f: ["-mllvm", "-disable-machine-sink"] for f in ("r9k_moe_prefill.hip", "r9k_moe_mid.hip", "r9k_moe_nvfp4.hip")}
+# Per-source additions. The prefill GEMMs interleave their MFMAs with LDS reads, DMA issue and conversions under
+# scheduling barriers; machine sinking would move the pure operations past the loop's wait/barrier branches into the
+# block that uses them and undo that order.
+FILE_FLAGS = {f: ["-mllvm", "-disable-machine-sink"]
+              for f in ("r9k_moe_prefill.hip", "r9k_moe_mid.hip", "r9k_moe_nvfp4.hip")}
 
 
 def hipcc() -> str:

@@ -289,14 +289,20 @@ void nv_launch(dim3 grid, hipStream_t st, long a, long as, long wq, long ws, lon
 // ------------------------------------------------------------------------------------------ prefill (tiles of 128)
 // Routed rows in blocks of 128 (a routing block of 128 or 256 rows covered by 1 or 2 workgroups along grid.y) x 128
 // output columns per workgroup; 4 waves in 2 x 2, each 64 rows x 64 columns = 4 x 4 tiles of the fp16 MFMA above.
-// K runs in 128-wide tiles through a ring of three LDS stages (activations 16 KB, codes 8 KB, scales 1 KB) filled by
-// direct global -> LDS DMA two K-tiles ahead of the MFMAs (every wave issues the same 7 DMA instructions a stage, so
-// the waits are fixed vmcnt counts; no compiler-tracked load sits in the loop). Each wave widens its 4 column tiles'
-// weights once per K-tile (codes and scales from LDS, as in the decode kernel) and reuses them over its 4 row tiles;
-// the activation rows are widened per row tile. Activation row pieces sit XOR-swizzled (16-byte piece p of row r at
-// position p ^ (r & 7)) so the 16 rows a fragment read touches land in different banks: the DMA lane that fills
-// position p of row r fetches piece p ^ (r & 7). Past K (a partial last K-tile) an activation piece is fetched from
-// the row's last valid piece; the weights' codes and scales there are zero, so those products are exact zeros.
+// K runs in 128-wide tiles through a ring of three LDS slots (activations 16 KB, codes 8 KB, scales 1 KB) filled by
+// direct global -> LDS DMA (every wave issues the same 7 DMA instructions a K-tile, so the waits are fixed vmcnt counts;
+// no compiler-tracked load sits in the loop). Each wave widens its 4 column tiles' weights once per K-tile (codes and
+// scales from LDS, as in the decode kernel) and reuses them over its 4 row tiles; the activation rows are widened per
+// row tile. Bound: the matrix pipe and, nearly as long, the widening's vector instructions (two conversions and a
+// multiply an MFMA, all at the full rate of 4 clocks a wave instruction). So they have to overlap within a wave: every
+// MFMA carries one conversion pair of the next row tile's activations and one of the next K-tile's weights. Widening a
+// K-tile's weights ahead of its MFMAs instead left that to the other wave of the SIMD. [17408, 5120], 2000 rows: 325 ->
+// 313 us (1.14 PFLOP/s, where a plain bf16 matrix product of 8192^3 reaches 1.21 on the same card; matrix pipe busy 55%
+// of the clocks); row-block groups on top, an L2-friendlier tile order, 0.7%: not kept.
+// Activation row pieces sit XOR-swizzled (16-byte piece p of row r at position p ^ (r & 7)) so the 16 rows a fragment
+// read touches land in different banks: the DMA lane that fills position p of row r fetches piece p ^ (r & 7). Past K
+// (a partial last K-tile) an activation piece is fetched from the row's last valid piece; the weights' codes and scales
+// there are zero, so those products are exact zeros.
 constexpr int PV_BM = 128, PV_BN = 128, PV_THREADS = 256;
 constexpr int PV_NS = 3;           // LDS stages
 constexpr int PV_DMA = 7;          // DMA instructions per wave and stage: 4 activation, 2 code, 1 scale

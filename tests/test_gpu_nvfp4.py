@@ -109,6 +109,14 @@ def test_nvfp4_linear(dev, M, N, Kd):
     check(O.bf16_bits(out), ref)
 
 
+@pytest.mark.parametrize("M,N,Kd", [(128, 16, 32), (129, 144, 128), (200, 128, 160), (256, 272, 256), (131, 128, 416),
+                                    (257, 144, 512), (128, 64, 640), (300, 128, 896)])
+def test_nvfp4_linear_prefill_k_tiles(dev, M, N, Kd):
+    """The prefill kernel's ring at 1 to 7 K-tiles, odd and even, full and partial: fewer than its slots, and each
+    parity of the double-buffered weights."""
+    test_nvfp4_linear(dev, M, N, Kd)
+
+
 @pytest.mark.parametrize("M", [31, 32, 33, 64, 65, 127])
 def test_nvfp4_linear_wide_decode_blocks(dev, M):
     """Long K (5 K-tiles and more a wave) at 32- and 64-row routing blocks, where at most two blocks are launched."""
