@@ -227,3 +227,28 @@ def test_tuned_table_lookup(tmp_path, monkeypatch):
     monkeypatch.setattr(tuned, "_TABLE", None)
     assert K.pick_cfg(1024, 2048, M=40, kind="mxfp4") == (0, 0, 0)
     monkeypatch.setattr(tuned, "_TABLE", None)
+
+
+def test_launch_extension_releases_the_gil():
+    """A C entry that waits (a launch on a full queue) must not hold up the other threads: usleep through the launch
+    extension in one thread, a short sleep in this one."""
+    import ctypes
+    import threading
+    import time
+    from r9700_vllm.kernels import moe as KM
+    call = (KM._native or KM._load_native()).call
+    usleep = ctypes.cast(ctypes.CDLL(None).usleep, ctypes.c_void_p).value
+    entered = threading.Event()
+
+    def wait():
+        entered.set()
+        call(usleep, 600_000)
+
+    t = threading.Thread(target=wait)
+    t.start()
+    entered.wait()
+    t0 = time.perf_counter()
+    time.sleep(0.05)
+    dt = time.perf_counter() - t0
+    t.join()
+    assert dt < 0.4, f"a 50 ms sleep took {dt:.2f} s beside a waiting entry"
