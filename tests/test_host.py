@@ -229,26 +229,29 @@ def test_tuned_table_lookup(tmp_path, monkeypatch):
     monkeypatch.setattr(tuned, "_TABLE", None)
 
 
-def test_launch_extension_releases_the_gil():
-    """A C entry that waits (a launch on a full queue) must not hold up the other threads: usleep through the launch
-    extension in one thread, a short sleep in this one."""
-    import ctypes
+def _beside(wait) -> bool:
+    """Whether this thread runs while another one is inside wait() (0.6 s): it starts the other one, sees it enter and
+    sleeps 50 ms long before wait() returns. The clock starts before the thread does: a wait() that keeps the GIL holds
+    this thread up in start() or entered.wait() already, not only in the sleep."""
     import threading
     import time
-    from r9700_vllm.kernels import moe as KM
-    call = (KM._native or KM._load_native()).call
-    usleep = ctypes.cast(ctypes.CDLL(None).usleep, ctypes.c_void_p).value
     entered = threading.Event()
-
-    def wait():
-        entered.set()
-        call(usleep, 600_000)
-
-    t = threading.Thread(target=wait)
+    t = threading.Thread(target=lambda: (entered.set(), wait()))
+    t0 = time.perf_counter()
     t.start()
     entered.wait()
-    t0 = time.perf_counter()
     time.sleep(0.05)
-    dt = time.perf_counter() - t0
+    beside = t.is_alive() and time.perf_counter() - t0 < 0.4
     t.join()
-    assert dt < 0.4, f"a 50 ms sleep took {dt:.2f} s beside a waiting entry"
+    return beside
+
+
+def test_launch_extension_releases_the_gil():
+    """A C entry that waits (a launch on a full queue) must not hold up the other threads: usleep through the launch
+    extension. The same wait with the GIL held (PyDLL) fails the check."""
+    import ctypes
+    call = (K._native or K._load_native()).call
+    usleep = ctypes.cast(ctypes.CDLL(None).usleep, ctypes.c_void_p).value
+    assert _beside(lambda: call(usleep, 600_000))
+    held = ctypes.PyDLL(None).usleep
+    assert not _beside(lambda: held(600_000))
