@@ -254,6 +254,13 @@ int r9k_dense_mxfp4_a8(long q, long ldq, long s, long tw, long wq, long ws, long
 int r9k_dense_nvfp4_qa(long x, long ldx, long wq, long ws, long wg, long out, long ldo, int M, int N, int K,
                        long stream);
 
+/* The GEMM of the same linear from 1 <= M <= 16 rows already quantised: q fp8 [M][K] (row stride ldq bytes, 16-byte
+ * aligned rows), s fp32 [M]; wq / ws / wg one native NVFP4 expert, out bf16 [M][N] (row stride ldo elements).
+ * r9k_moe_nvfp4a8's values over identity tables, bit for bit. 2 (nothing launched) for M > 16, K % 128, N % 16 or an
+ * unaligned base; -3 bad argument, -6 launch error. */
+int r9k_dense_nvfp4_a8(long q, long ldq, long s, long wq, long ws, long wg, long out, long ldo, int M, int N, int K,
+                       long stream);
+
 /* Load-time NVFP4 -> MXFP4 with MSE-searched block exponents (the reference does this with torch:
  * r9700_vllm/quant/nvfp4.py:39-90). packed u8 [N][K/2], s16 e4m3 [N][K/16], row_div fp32 [N] -> out_packed u8
  * [N][K/2], out_e8m0 u8 [N][K/32] (checkpoint layout). -2 K % 32, -3 bad pointer / alignment, -6 launch error. */
