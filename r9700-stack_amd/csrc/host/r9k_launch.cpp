@@ -1,7 +1,11 @@
 // r9k_launch.cpp -- the Python bindings' launch helpers as a CPython extension (r9700_vllm/kernels/_r9k_launch.so):
 //
-//   call(address, *args) -> int      a libr9k C entry: a tensor passes its data pointer, None 0, an int its value
+//   call(spec, *args) -> int         a libr9k C entry; spec is its address (8 bytes) and one kind letter an argument
 //   empty(like, dtype, *sizes)       torch.empty(sizes) of a torch.dtype on like's device
+//
+// Kinds: p a device pointer (a tensor passes its data pointer, an int itself), o the same or None (0), l a long, i an int.
+// Numbers go through __index__ and wrap to their C width, as ctypes converts them: a 0-d integer tensor in an l or i
+// position is its value, never its address, and None is a number nowhere.
 //
 // A decode step is a handful of launches of a few microseconds, and its host side was bound by the bindings: a ctypes
 // call converts each argument by its argtype (a 20-argument launch with its data_ptr() calls ~5 us beside the ~3 us the
@@ -18,6 +22,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstring>
 #include <utility>
 
 #if !defined(__x86_64__)
@@ -43,37 +48,55 @@ int dispatch(size_t n, long fn, const long* v) {
   return -1000;
 }
 
+// A number argument as ctypes takes it: anything with __index__, wrapped to 64 bits.
+bool number(PyObject* a, long* v) {
+  PyObject* n = PyNumber_Index(a);
+  if (!n) return false;
+  *v = (long)PyLong_AsUnsignedLongMask(n);
+  Py_DECREF(n);
+  return !(*v == -1 && PyErr_Occurred());
+}
+
 PyObject* py_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  if (nargs < 2 || nargs - 1 > MAX_ARGS) {
-    PyErr_Format(PyExc_TypeError, "call(address, *args): 1 to %d arguments, got %zd", MAX_ARGS, nargs - 1);
+  if (nargs < 1 || !PyBytes_Check(args[0]) || PyBytes_GET_SIZE(args[0]) <= (Py_ssize_t)sizeof(long)) {
+    PyErr_SetString(PyExc_TypeError, "call(spec, *args): spec is an entry's address and its argument kinds, as bytes");
     return nullptr;
   }
-  const long fn = PyLong_AsLong(args[0]);
-  if (fn == -1 && PyErr_Occurred()) return nullptr;
+  const char* kind = PyBytes_AS_STRING(args[0]) + sizeof(long);
+  const Py_ssize_t want = PyBytes_GET_SIZE(args[0]) - (Py_ssize_t)sizeof(long);
+  if (want > MAX_ARGS || nargs - 1 != want) {
+    PyErr_Format(PyExc_TypeError, "call: the entry takes %zd arguments (at most %d), got %zd", want, MAX_ARGS, nargs - 1);
+    return nullptr;
+  }
+  long fn;
+  std::memcpy(&fn, PyBytes_AS_STRING(args[0]), sizeof fn);
   if (fn == 0) {
     PyErr_SetString(PyExc_ValueError, "call: null entry address");
     return nullptr;
   }
   long v[MAX_ARGS];
-  for (Py_ssize_t i = 1; i < nargs; i++) {
-    PyObject* a = args[i];
-    if (PyLong_Check(a)) {
-      v[i - 1] = PyLong_AsLong(a);
-      if (v[i - 1] == -1 && PyErr_Occurred()) return nullptr;
-    } else if (a == Py_None) {
-      v[i - 1] = 0;
-    } else if (THPVariable_Check(a)) {
-      v[i - 1] = reinterpret_cast<long>(THPVariable_Unpack(a).data_ptr());
-    } else {
-      PyErr_Format(PyExc_TypeError, "call: argument %zd is a %s, not an int, a tensor or None", i, Py_TYPE(a)->tp_name);
+  for (Py_ssize_t i = 0; i < want; i++) {
+    PyObject* a = args[i + 1];
+    int over = 0;
+    if (PyLong_CheckExact(a) && (v[i] = PyLong_AsLongAndOverflow(a, &over), over == 0)) {
+      if (kind[i] == 'i') v[i] = (int)v[i];
+    } else if ((kind[i] == 'p' || kind[i] == 'o') && THPVariable_Check(a)) {
+      v[i] = reinterpret_cast<long>(THPVariable_Unpack(a).data_ptr());
+    } else if (kind[i] == 'o' && a == Py_None) {
+      v[i] = 0;
+    } else if (!number(a, &v[i])) {
+      if (PyErr_ExceptionMatches(PyExc_TypeError))
+        PyErr_Format(PyExc_TypeError, "call: argument %zd (kind %c) is a %s", i + 1, kind[i], Py_TYPE(a)->tp_name);
       return nullptr;
+    } else if (kind[i] == 'i') {
+      v[i] = (int)v[i];
     }
   }
   // without the GIL, as ctypes calls it: a launch waits while its queue is full, and another thread may have to run first
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = dispatch<1>((size_t)nargs - 1, fn, v);
+  rc = dispatch<1>((size_t)want, fn, v);
   Py_END_ALLOW_THREADS
   return PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
@@ -99,7 +122,7 @@ PyObject* py_empty(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 PyMethodDef kMethods[] = {
     {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_call)), METH_FASTCALL,
-     "call(address, *args) -> int: a libr9k entry on tensors (their data pointers), ints and None (0)"},
+     "call(spec, *args) -> int: a libr9k entry, its address and argument kinds in spec, on tensors, numbers and None"},
     {"empty", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_empty)), METH_FASTCALL,
      "empty(like, dtype, *sizes) -> an uninitialised tensor on like's device"},
     {nullptr, nullptr, 0, nullptr}};

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from dataclasses import dataclass
 
 import torch
@@ -26,71 +27,56 @@ def _lib_path() -> str:
     return os.environ.get("R9K_LIB") or os.path.join(os.path.dirname(__file__), "libr9k.so")
 
 
+# The C entries' arguments, a letter each: p a device pointer, o a pointer that may be left out (0), l a long (strides in
+# bytes or elements, the stream), i an int. ctypes and the launch extension (_call) both read them from here.
+_SIGS: dict = {}
+
+
+def bind(L: ctypes.CDLL, name: str, sig: str, restype=ctypes.c_int) -> None:
+    """Declare entry `name` of `L` with the argument kinds `sig` (spaces only group them)."""
+    sig = sig.replace(" ", "")
+    fn = getattr(L, name)
+    fn.argtypes = [ctypes.c_int if c == "i" else ctypes.c_long for c in sig]
+    fn.restype = restype
+    _SIGS[name] = sig
+
+
 def lib() -> ctypes.CDLL:
     """The kernel library (lazy, process-global). Raises OSError when libr9k.so is missing: there is no fallback."""
     global _LIB
     if _LIB is None:
         L = ctypes.CDLL(_lib_path())
-        i, l = ctypes.c_int, ctypes.c_long
-        L.r9k_moe_mxfp4a8.restype = i
-        L.r9k_moe_mxfp4a8.argtypes = [l] * 12 + [i] * 9 + [l]
-        L.r9k_moe_mxfp4a8_f.restype = i
-        L.r9k_moe_mxfp4a8_f.argtypes = [i] + [l] * 12 + [i] * 9 + [l]
-        L.r9k_moe_nvfp4a8.restype = i
-        L.r9k_moe_nvfp4a8.argtypes = [l] * 12 + [i] * 9 + [l]
-        L.r9k_moe_4bit_prefill.restype = i
-        L.r9k_moe_4bit_prefill.argtypes = [i] + [l] * 12 + [i] * 6 + [l]
-        L.r9k_moe_prefill_bm.restype = i
-        L.r9k_moe_prefill_bm.argtypes = [i]
-        L.r9k_moe_prefill_bk.restype = i
-        L.r9k_moe_prefill_bk.argtypes = [i]
-        L.r9k_quant_rows_fp8.restype = i
-        L.r9k_quant_rows_fp8.argtypes = [l] * 3 + [i] * 3 + [l]
-        L.r9k_silu_mul_quant_fp8.restype = i
-        L.r9k_silu_mul_quant_fp8.argtypes = [l] * 3 + [i] * 2 + [l]
-        L.r9k_quant_rows_fp8_gate.restype = i
-        L.r9k_quant_rows_fp8_gate.argtypes = [l] * 5 + [i] * 4 + [l]
-        L.r9k_moe_sum.restype = i
-        L.r9k_moe_sum.argtypes = [l] * 3 + [i] * 3 + [l] * 3
-        L.r9k_moe_topk.restype = i
-        L.r9k_moe_topk.argtypes = [l, i, l, l, i, i, i, i, l]
-        L.r9k_moe_topk_quant.restype = i
-        L.r9k_moe_topk_quant.argtypes = [l, i, l, l, i, i, i, i, l, l, i, l, l, l]
-        L.r9k_moe_align.restype = i
-        L.r9k_moe_align.argtypes = [l, i, i, i, l, l, l, l, l, l]
-        L.r9k_moe_align_live.restype = i
-        L.r9k_moe_align_live.argtypes = [l, i, i, i, l, l, l, l, l, l]
-        L.r9k_moe_align_split.restype = i
-        L.r9k_moe_align_split.argtypes = [l, i, i, i, i, l, l, l, i, l, l, l, l, l, l]
-        L.r9k_moe_align_scratch_ints.restype = l
-        L.r9k_moe_align_noalloc.restype = i
-        L.r9k_moe_align_noalloc.argtypes = [l, i, i, i, l, l, l, l]
-        L.r9k_moe_align_noalloc_max_ints.restype = l
-        L.r9k_moe_align_noalloc_max_ints.argtypes = []
-        L.r9k_moe_pick_blocks.restype = i
-        L.r9k_moe_pick_blocks.argtypes = [l, l, i, i, i, l]
-        L.r9k_moe_align_scratch_ints.argtypes = [i, i]
-        L.r9k_nvfp4_to_mxfp4.restype = i
-        L.r9k_nvfp4_to_mxfp4.argtypes = [l] * 5 + [i] * 2 + [l]
-        L.r9k_quantize_mxfp4_search.restype = i
-        L.r9k_quantize_mxfp4_search.argtypes = [l] * 3 + [i] * 2 + [l]
-        L.r9k_mxfp4_prep.restype = i
-        L.r9k_mxfp4_prep.argtypes = [l] * 4 + [i] * 3 + [l]
-        L.r9k_fold_supported.restype = i
-        L.r9k_moe_down_sum.restype = i
-        L.r9k_dense_mxfp4_qa.restype = i
-        L.r9k_dense_mxfp4_qa.argtypes = [l] * 6 + [i] * 3 + [l]
-        L.r9k_dense_mxfp4_a8.restype = i
-        L.r9k_dense_nvfp4_qa.restype = i
-        L.r9k_dense_nvfp4_qa.argtypes = [l] * 7 + [i] * 3 + [l]
-        L.r9k_dense_mxfp4_a8.argtypes = [l] * 8 + [i] * 3 + [l]
-        L.r9k_dense_nvfp4_a8.restype = i
-        L.r9k_dense_nvfp4_a8.argtypes = [l] * 8 + [i] * 3 + [l]
-        L.r9k_moe_down_sum.argtypes = [l] * 10 + [i] * 5 + [l]
-        L.r9k_moe_stream.restype = i
-        L.r9k_moe_stream.argtypes = [i] + [l] * 11 + [i] * 6 + [l]
-        L.r9k_moe_stream_layer.restype = i
-        L.r9k_moe_stream_layer.argtypes = [l] * 13 + [i] * 6 + [l]
+        gemm = "pppp p p ppp o ll"          # a, as, wq, ws, wref / wg, c, the tables, topk_w, two expert strides
+        bind(L, "r9k_moe_mxfp4a8", gemm + "iii iii iii l")
+        bind(L, "r9k_moe_mxfp4a8_f", "i po pp p p ppp o ll iii iii iii l")
+        bind(L, "r9k_moe_nvfp4a8", gemm + "iii iii iii l")
+        bind(L, "r9k_moe_4bit_prefill", "i" + gemm + "iii iii l")
+        bind(L, "r9k_moe_prefill_bm", "i")
+        bind(L, "r9k_moe_prefill_bk", "i")
+        bind(L, "r9k_quant_rows_fp8", "ppp iii l")
+        bind(L, "r9k_silu_mul_quant_fp8", "ppp ii l")
+        bind(L, "r9k_quant_rows_fp8_gate", "ppppp iiii l")
+        bind(L, "r9k_moe_sum", "pop iii lll")
+        bind(L, "r9k_moe_topk", "pi pp iiii l")
+        bind(L, "r9k_moe_topk_quant", "pi pp iiii pli pp l")
+        bind(L, "r9k_moe_align", "p iii ppp pl l")
+        bind(L, "r9k_moe_align_live", "p iii ppp pl l")
+        bind(L, "r9k_moe_align_split", "p iii i ppp i ppp pl l")
+        bind(L, "r9k_moe_align_scratch_ints", "ii", ctypes.c_long)
+        bind(L, "r9k_moe_align_noalloc", "p iii ppp l")
+        bind(L, "r9k_moe_align_noalloc_max_ints", "", ctypes.c_long)
+        bind(L, "r9k_moe_pick_blocks", "pp iii l")
+        bind(L, "r9k_nvfp4_to_mxfp4", "ppp pp ii l")
+        bind(L, "r9k_quantize_mxfp4_search", "p pp ii l")
+        bind(L, "r9k_mxfp4_prep", "oooo iii l")
+        bind(L, "r9k_fold_supported", "")
+        bind(L, "r9k_dense_mxfp4_qa", "pl pp pl iii l")
+        bind(L, "r9k_dense_mxfp4_a8", "pl po pp pl iii l")
+        bind(L, "r9k_dense_nvfp4_qa", "pl ppp pl iii l")
+        bind(L, "r9k_dense_nvfp4_a8", "pl p ppp pl iii l")
+        bind(L, "r9k_moe_down_sum", "ppp ppl ol pl iiiii l")
+        bind(L, "r9k_moe_stream", "i pp pp po ppp o l iii iii l")
+        bind(L, "r9k_moe_stream_layer", "pp pppp p ppp p ll iii iii l")
         assert L.r9k_moe_block() == MOE_BLOCK
         _LIB = L
     return _LIB
@@ -106,11 +92,11 @@ def atiled_supported() -> bool:
     return hasattr(lib(), "r9k_moe_4bit_prefill_at")
 
 
-# Launches go through a CPython extension (csrc/host/r9k_launch.cpp, built beside libr9k.so): `_call` passes tensors as
-# their data pointers and None as 0, `_empty` allocates. Measured on the MI355X host, per use: a 20-argument ctypes call
+# Launches go through a CPython extension (csrc/host/r9k_launch.cpp, built beside libr9k.so): `_call` passes tensors in
+# pointer positions as their data pointers, `_empty` allocates. Measured on the MI355X host, per use: a 20-argument ctypes call
 # with its data_ptr() calls ~5 us beyond the launch against ~1; torch.empty 1.7 us against 1.0; the public
 # torch.cuda.current_stream() 2.9 us against 0.2 for the raw stream of the current device.
-_ADDR: dict = {}
+_ENTRIES: dict = {}                                            # name -> address and kinds, as the extension reads them
 _native = None
 
 
@@ -126,12 +112,17 @@ def _load_native():
     return mod
 
 
+def _spec(fn, sig: str) -> bytes:
+    """What the extension's call() takes for a C function: its address and its arguments' kinds."""
+    return struct.pack("=q", ctypes.cast(fn, ctypes.c_void_p).value) + sig.encode()
+
+
 def _call(name: str, *args) -> int:
-    """libr9k's C entry `name` (long and int arguments only) on tensors, ints and None."""
-    a = _ADDR.get(name)
-    if a is None:
-        a = _ADDR[name] = ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
-    return (_native or _load_native()).call(a, *args)
+    """libr9k's C entry `name` on tensors, numbers and, where its signature says so, None."""
+    e = _ENTRIES.get(name)
+    if e is None:
+        e = _ENTRIES[name] = _spec(getattr(lib(), name), _SIGS[name])
+    return (_native or _load_native()).call(e, *args)
 
 
 def _empty(like: torch.Tensor, dtype: torch.dtype, *sizes: int) -> torch.Tensor:

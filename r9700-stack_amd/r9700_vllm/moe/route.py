@@ -43,15 +43,12 @@ def lib() -> ctypes.CDLL:
         L = KM.lib()
         if not hasattr(L, "r9k_moe_route"):
             raise RuntimeError("libr9k.so has no r9k_moe_route (rebuild r9700-stack_amd)")
-        i, l = ctypes.c_int, ctypes.c_long
-        common = [l, i] + [l] * 6 + [i] * 5          # logits, ldl, w, ids, sorted, expert_ids, ntpp, scratch, M..blk
-        L.r9k_moe_route.argtypes, L.r9k_moe_route.restype = common + [l], i
-        L.r9k_moe_route_quant.argtypes = common + [l, l, i, l, l, l]
-        L.r9k_moe_route_quant.restype = i
-        L.r9k_moe_route_dual.argtypes = common + [l, l, i, l, l, i, l, l, l, i, l]
-        L.r9k_moe_route_dual.restype = i
-        L.r9k_moe_route_max_experts.restype = i
-        L.r9k_moe_route_max_topk.restype = i
+        common = "pi pp ppp p iii ii"                # logits, ldl, w, ids, the tables, scratch, M..blk
+        KM.bind(L, "r9k_moe_route", common + "l")
+        KM.bind(L, "r9k_moe_route_quant", common + "pli pp l")
+        KM.bind(L, "r9k_moe_route_dual", common + "oli oo i ppp i l")
+        KM.bind(L, "r9k_moe_route_max_experts", "")
+        KM.bind(L, "r9k_moe_route_max_topk", "")
         _limits[:] = L.r9k_moe_route_max_experts(), L.r9k_moe_route_max_topk()
         _bound = L
     return _bound
@@ -77,6 +74,12 @@ def scratch_ints(E: int) -> int:
     return 2 * E + 1
 
 
+def _call(name: str, *args) -> int:
+    if _bound is None:
+        lib()                                        # declares the routing entries
+    return KM._call(name, *args)
+
+
 def _launch(quant_x, logits, topk, renorm, blk, sorted_ids, expert_ids, ntpp, scratch):
     """One routing launch; with quant_x also the fp8 quant of that input. Returns (rc, w, ids, xq, xs)."""
     M, E = logits.shape
@@ -85,11 +88,11 @@ def _launch(quant_x, logits, topk, renorm, blk, sorted_ids, expert_ids, ntpp, sc
     head = (logits, logits.stride(0), w, ids, sorted_ids, expert_ids, ntpp, scratch, M, E, topk, int(bool(renorm)), blk)
     st = KM._stream()
     if quant_x is None:
-        return KM._call("r9k_moe_route", *head, st), w, ids, None, None
+        return _call("r9k_moe_route", *head, st), w, ids, None, None
     H = quant_x.shape[1]
     xq = KM._empty(logits, torch.float8_e4m3fn, M, H)
     xs = KM._empty(logits, torch.float32, M)
-    rc = KM._call("r9k_moe_route_quant", *head, quant_x, quant_x.stride(0), H, xq, xs, st)
+    rc = _call("r9k_moe_route_quant", *head, quant_x, quant_x.stride(0), H, xq, xs, st)
     return rc, w, ids, xq, xs
 
 
@@ -145,7 +148,7 @@ def moe_route_dual(logits: torch.Tensor, topk: int, renorm: bool, blk: int, sort
         xq = torch.empty((M, H), dtype=torch.float8_e4m3fn, device=dev)
         xs = torch.empty((M,), dtype=torch.float32, device=dev)
         xa = (x, x.stride(0), H, xq, xs)
-    rc = KM._call("r9k_moe_route_dual", logits, logits.stride(0), w, ids, sorted_ids, expert_ids, ntpp, scratch, M, E,
+    rc = _call("r9k_moe_route_dual", logits, logits.stride(0), w, ids, sorted_ids, expert_ids, ntpp, scratch, M, E,
                   topk, int(renorm), blk, *xa, big_blk, sorted_big, expert_big, ntpp_big, min_rows, KM._stream())
     if rc:
         raise RuntimeError(f"r9k_moe_route_dual failed ({rc}) M={M} E={E} topk={topk} blk={blk} big={big_blk}")

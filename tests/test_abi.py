@@ -23,6 +23,22 @@ def test_header_symbols_exported():
     assert not missing, missing
 
 
+def test_signatures_match_the_header():
+    """The argument kinds that ctypes and the launch extension convert by: int parameters are i, strides, counts and the
+    stream l, every other long a pointer (p, or o when the entry takes 0 for it)."""
+    from r9700_vllm.moe import route
+    route.lib()
+    src = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "r9k.h")).read(), flags=re.S)
+    protos = dict(re.findall(r"^\s*(?:int|long)\s+(r9k_\w+)\s*\(([^)]*)\)", src, flags=re.M))
+    assert len(K._SIGS) >= 30
+    for name, sig in K._SIGS.items():
+        params = [p.split() for p in protos[name].split(",") if p.strip() != "void"]
+        number = [t == "int" or n in ("stream", "scratch_ints") or n.startswith("ld") or n.endswith("_estride")
+                  for t, n in params]
+        want = "".join("i" if t == "int" else ("l" if num else "p") for (t, n), num in zip(params, number))
+        assert sig.replace("o", "p") == want, (name, sig, want)
+
+
 def test_python_binding_contract():
     L = K.lib()
     assert L.r9k_moe_block() == 16

@@ -229,6 +229,43 @@ def test_tuned_table_lookup(tmp_path, monkeypatch):
     monkeypatch.setattr(tuned, "_TABLE", None)
 
 
+@pytest.fixture
+def entry(monkeypatch):
+    """A stand-in for a libr9k entry behind kernels.moe._call: records its four C arguments (long, long, int, long)."""
+    import ctypes
+    got = []
+    proto = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_long, ctypes.c_long, ctypes.c_int, ctypes.c_long)
+    cb = proto(lambda *a: got.append(a) or 7)
+    monkeypatch.setitem(K._ENTRIES, "stand_in", K._spec(cb, "plio"))
+    return got, lambda *a: K._call("stand_in", *a), cb
+
+
+def test_launch_numbers_convert_as_ctypes_did(entry):
+    """A number position takes anything with __index__ by its value -- numpy integers, bools, 0-d integer tensors (never
+    their address) -- wrapped to its C width; a pointer position a tensor's address or an address."""
+    got, call, _ = entry
+    t = torch.zeros(3)
+    assert call(t, np.int64(40), torch.tensor(5), None) == 7
+    assert got[-1] == (t.data_ptr(), 40, 5, 0)
+    call(t.data_ptr(), True, np.uint8(200), t)
+    assert got[-1] == (t.data_ptr(), 1, 200, t.data_ptr())
+    call(0, torch.tensor(-3), torch.tensor([9], dtype=torch.int32), 0)
+    assert got[-1] == (0, -3, 9, 0)
+    call(torch.nn.Parameter(t, requires_grad=False), (1 << 64) + 2, (1 << 32) + 6, 0)
+    assert got[-1] == (t.data_ptr(), 2, 6, 0)
+
+
+def test_launch_refuses_what_is_no_argument(entry):
+    """None where a tensor is required, non-integers, tensors of several values in a number position, a wrong count."""
+    got, call, _ = entry
+    t = torch.zeros(3)
+    for bad in ((None, 1, 2, 0), (t, None, 2, 0), (t, 1, None, 0), (t, 1.0, 2, 0), (t, 1, torch.tensor(2.0), 0),
+                (t, 1, torch.zeros(2, dtype=torch.int32), 0), (t, 1, "2", 0), ([t], 1, 2, 0), (t, 1, 2), (t, 1, 2, 0, 0)):
+        with pytest.raises(TypeError):
+            call(*bad)
+    assert not got
+
+
 def _beside(wait) -> bool:
     """Whether this thread runs while another one is inside wait() (0.6 s): it starts the other one, sees it enter and
     sleeps 50 ms long before wait() returns. The clock starts before the thread does: a wait() that keeps the GIL holds
@@ -251,7 +288,7 @@ def test_launch_extension_releases_the_gil():
     extension. The same wait with the GIL held (PyDLL) fails the check."""
     import ctypes
     call = (K._native or K._load_native()).call
-    usleep = ctypes.cast(ctypes.CDLL(None).usleep, ctypes.c_void_p).value
+    usleep = K._spec(ctypes.CDLL(None).usleep, "i")
     assert _beside(lambda: call(usleep, 600_000))
     held = ctypes.PyDLL(None).usleep
     assert not _beside(lambda: held(600_000))
