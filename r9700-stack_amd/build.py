@@ -3,7 +3,8 @@
     python r9700-stack_amd/build.py            # -> r9700-stack_amd/r9700_vllm/kernels/libr9k.so
 
 Every `csrc/*.hip` is compiled for gfx950 only and linked into one shared library exporting the C-ABI declared in
-include/r9k.h, and the bindings' launch helpers (csrc/host) become `_r9k_launch.so` beside it. Objects go to `_build/` next to this file (not tracked).
+include/r9k.h. The bindings' launch helpers (csrc/host) become `_r9k_launch.<CPython ABI tag>.so` beside it. Objects go to
+`_build/` next to this file (not tracked).
 """
 from __future__ import annotations
 
@@ -13,11 +14,12 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "r9700_vllm", "kernels", "libr9k.so")
-LAUNCH = os.path.join(HERE, "r9700_vllm", "kernels", "_r9k_launch.so")
+LAUNCH = os.path.join(HERE, "r9700_vllm", "kernels", "_r9k_launch" + sysconfig.get_config_var("EXT_SUFFIX"))
 BUILD = os.path.join(HERE, "_build")
 
 ARCH = "gfx950"
@@ -52,8 +54,6 @@ def _compile(src: str) -> str:
 
 def build_launch(out: str = LAUNCH) -> str:
     """The bindings' launch helpers (csrc/host/r9k_launch.cpp): a CPython extension over torch's C++ API, host code only."""
-    import sysconfig
-
     import torch
     root = os.path.dirname(torch.__file__)
     inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
@@ -61,7 +61,8 @@ def build_launch(out: str = LAUNCH) -> str:
     lib = os.path.join(root, "lib")
     tmp = out + ".tmp"
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in inc),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DR9K_TORCH="{torch.__version__}"',
+           *(f"-I{d}" for d in inc),
            os.path.join(CSRC, "host", "r9k_launch.cpp"), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode:

@@ -1,7 +1,8 @@
-// r9k_launch.cpp -- the Python bindings' launch helpers as a CPython extension (r9700_vllm/kernels/_r9k_launch.so):
+// r9k_launch.cpp -- the Python bindings' launch helpers as a CPython extension (r9700_vllm/kernels/_r9k_launch.*.so):
 //
 //   call(spec, *args) -> int         a libr9k C entry; spec is its address (8 bytes) and one kind letter an argument
 //   empty(like, dtype, *sizes)       torch.empty(sizes) of a torch.dtype on like's device
+//   TORCH                            the torch version it was built against
 //
 // Kinds: p a device pointer (a tensor passes its data pointer, an int itself), o the same or None (0), l a long, i an int.
 // Numbers go through __index__ and wrap to their C width, as ctypes converts them: a 0-d integer tensor in an l or i
@@ -132,4 +133,8 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_r9k_launch", "Launch helpers of 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__r9k_launch(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__r9k_launch(void) {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "TORCH", R9K_TORCH)) Py_CLEAR(m);
+  return m;
+}

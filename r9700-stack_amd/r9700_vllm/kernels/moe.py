@@ -10,8 +10,10 @@ plus its 64 exponent bytes. Everything here launches on torch's current stream a
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import struct
+import sysconfig
 from dataclasses import dataclass
 
 import torch
@@ -42,10 +44,12 @@ def bind(L: ctypes.CDLL, name: str, sig: str, restype=ctypes.c_int) -> None:
 
 
 def lib() -> ctypes.CDLL:
-    """The kernel library (lazy, process-global). Raises OSError when libr9k.so is missing: there is no fallback."""
+    """The kernel library (lazy, process-global). Raises OSError when libr9k.so or the launch extension beside it cannot
+    be loaded: there is no fallback."""
     global _LIB
     if _LIB is None:
         L = ctypes.CDLL(_lib_path())
+        _load_native()
         gemm = "pppp p p ppp o ll"          # a, as, wq, ws, wref / wg, c, the tables, topk_w, two expert strides
         bind(L, "r9k_moe_mxfp4a8", gemm + "iii iii iii l")
         bind(L, "r9k_moe_mxfp4a8_f", "i po pp p p ppp o ll iii iii iii l")
@@ -100,14 +104,24 @@ _ENTRIES: dict = {}                                            # name -> address
 _native = None
 
 
+def launch_path() -> str:
+    """The launch extension of this interpreter (its name carries the CPython ABI tag)."""
+    return os.path.join(os.path.dirname(__file__), "_r9k_launch" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
 def _load_native():
+    """The launch extension; OSError when it is missing, does not load or was built for another torch. lib() loads it too,
+    so whoever asks for the library knows that its entries can be called."""
     global _native
-    lib()
-    import importlib.util
-    path = os.path.join(os.path.dirname(__file__), "_r9k_launch.so")
-    spec = importlib.util.spec_from_file_location("_r9k_launch", path)
-    mod = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(mod)
+    path = launch_path()
+    try:
+        spec = importlib.util.spec_from_file_location("_r9k_launch", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+    except ImportError as e:
+        raise OSError(f"cannot load the launch extension {path}: {e}") from e
+    if mod.TORCH != torch.__version__:
+        raise OSError(f"{path} was built for torch {mod.TORCH}, this is {torch.__version__}: rebuild r9700-stack_amd")
     _native = mod
     return mod
 

@@ -47,6 +47,38 @@ def test_python_binding_contract():
     assert K.prefill_block(17) == 64 and L.r9k_moe_prefill_bm(20) == -1 and L.r9k_moe_prefill_bk(-1) == -1
 
 
+def test_unavailable_without_the_launch_extension(monkeypatch, tmp_path):
+    """lib() and every availability check fail without the launch extension, with one that does not load and with one of
+    another torch -- before the first step, not at it."""
+    import pytest
+    from r9700_vllm import router
+    from r9700_vllm.moe import route, shared
+    good = K.launch_path()
+    junk = tmp_path / "junk.so"
+    junk.write_bytes(b"no ELF")
+
+    def unload():
+        monkeypatch.setattr(K, "_LIB", None)
+        monkeypatch.setattr(K, "_native", None)
+        monkeypatch.setattr(route, "_bound", None)
+
+    def refused(match):
+        unload()
+        with pytest.raises(OSError, match=match):
+            K.lib()
+        assert not route.available() and not shared.available() and not router.available()
+
+    for path in (tmp_path / "absent.so", junk):
+        monkeypatch.setattr(K, "launch_path", lambda p=path: str(p))
+        refused("launch extension")
+    monkeypatch.setattr(K, "launch_path", lambda: good)
+    monkeypatch.setattr(K.torch, "__version__", "0.0.0")
+    refused("built for torch")
+    monkeypatch.undo()
+    unload()
+    assert route.available() and shared.available() and router.available()
+
+
 def test_shape_errors_before_launch():
     L = K.lib()
     z = 0
