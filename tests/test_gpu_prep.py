@@ -42,6 +42,26 @@ def test_prep_output_sizes(dev):
     assert torch.equal(long[:, :-1].cpu(), K.pack_scales(e8)) and bool((long[:, -1] == 7).all())
 
 
+def test_nvfp4_conversion_of_strided_tensors_stays_chunked(dev):
+    """Codes and scales that lie in wider buffers: the bytes of the contiguous conversion, and no copy of the whole
+    tensor (a chunk's rows at a time)."""
+    g = torch.Generator().manual_seed(11)
+    N, Kd = 8192, 2048
+    p = torch.randint(0, 256, (N, Kd // 2 + 64), generator=g, dtype=torch.uint8).to(dev)
+    s = (torch.randn(N, Kd // 16 + 32, generator=g).abs() * 20).clamp(2 ** -9, 448).to(torch.float8_e4m3fn).to(dev)
+    pv, sv, div = p[:, : Kd // 2], s[:, : Kd // 16], torch.full((N,), 448.0, device=dev)
+    want = NV.nvfp4_to_mxfp4(pv.contiguous(), sv.contiguous(), div)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    got = NV.nvfp4_to_mxfp4(pv, sv, div, rows_per_chunk=512)
+    extra = torch.cuda.max_memory_allocated() - base
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    outputs = N * Kd // 2 + N * Kd // 32
+    chunk = 512 * (Kd // 2 + Kd // 16)
+    assert extra <= outputs + 3 * chunk + (1 << 20), (extra, outputs, chunk)      # two chunks may be alive, and their rounding
+
+
 @pytest.mark.parametrize("rd", [1.0, 448.0, 2688.0 / 3.7, 1e30, 1e-30, 3.3e38])
 def test_nvfp4_search_branches(dev, rd):
     """Uniform blocks, every scale byte (zero, subnormal, negative, NaN), one-magnitude and all-zero blocks, groups whose

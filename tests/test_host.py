@@ -229,6 +229,16 @@ def test_tuned_table_lookup(tmp_path, monkeypatch):
     monkeypatch.setattr(tuned, "_TABLE", None)
 
 
+def test_conversion_launch_rows():
+    """One launch for tensors the conversion reads where they are; chunks for strided ones and for those elsewhere."""
+    from r9700_vllm.quant.nvfp4 import _launch_rows
+    cpu, meta = torch.device("cpu"), torch.device("meta")
+    p, s = torch.zeros(5000, 64, dtype=torch.uint8), torch.zeros(5000, 8, dtype=torch.uint8)
+    assert _launch_rows(p, s, cpu, 2048) == 5000 and _launch_rows(p[:0], s[:0], cpu, 2048) == 1
+    for a, b in ((p[:, ::2], s), (p, s[:, :4]), (p.to(meta), s), (p, s.to(meta))):
+        assert _launch_rows(a, b, cpu, 2048) == 2048
+
+
 @pytest.fixture
 def entry(monkeypatch):
     """A stand-in for a libr9k entry behind kernels.moe._call: records its four C arguments (long, long, int, long)."""
