@@ -25,6 +25,7 @@ import torch
 from .._compat import vllm_available
 from ..kernels import moe as K
 from . import route
+from .cache import is_host
 
 ZERO_DOWN = os.environ.get("R9K_MOE_ZERO_DOWN", "0") == "1"
 # R9K_MOE_FUSE=1: at decode (MT == 1) the activation runs in the gate_up GEMM's epilogue and the per-row fp8 quant in
@@ -225,6 +226,11 @@ class R9700Mxfp4Experts(_experts_base()):
             (h1, h2), (c1, c2) = cache.hot(), cache.cold()
             need_cold = numel > cache.no_cold_limit
             staged = need_cold and cache.stage is not None
+            if need_cold and not staged and big is None:
+                # weights in host memory: the decode kernel, which reads each of their bytes once a routing block (the
+                # LDS-ring kernel re-reads a ring of stages past a workgroup's last step, here over the host link). The
+                # resident experts' pass takes it too: a row's bits do not depend on where its expert lies
+                pf_gate = pf_down = None
             if cache.fused:
                 # with staging the cold pass gets its tables from the stage map below, not from the host map; the
                 # same launch quantises the input unless the router already did
@@ -257,10 +263,15 @@ class R9700Mxfp4Experts(_experts_base()):
                 layer._r9k_dual_blk = bc[1] if dual_ok else 0
             # the LDS-ring kernel's 64- / 128-row blocks (small experts), unless the router built this step's tables
             mid = K.pick_mid_block(numel, E, K1, K2) if plain and not K.down_sum_fits(numel, N2, K2) else None
+            host = (mid is not None or pf_gate is not None) and (is_host(w1) or is_host(w2))
+            if host:                                         # host-offloaded weights without a cache: as its cold pass
+                mid = None
+                if big is None:
+                    pf_gate = pf_down = None
             if mid is not None and route.take(layer, topk_ids, blk, numel) is not None:
                 mid = None
             split = (plain and mid is None and K.split_wanted(numel, E, K1, K2)
-                     and not (big is not None and K.small_experts(K1, K2)))
+                     and (host or not (big is not None and K.small_experts(K1, K2))))
             if mid is not None:
                 pf_gate = pf_down = mid[0]
                 blk = mid[1]

@@ -377,6 +377,77 @@ def test_cached_layer_equals_resident_layer(dev, T):
         assert same
 
 
+@pytest.mark.parametrize("stage", [False, True])
+def test_cached_layer_at_64_row_blocks(dev, monkeypatch, stage):
+    """32 rows an expert and K % 128 != 0 (64-row routing blocks). A pass over host memory, and the resident pass beside
+    it, run on the decode kernel; with the cold experts staged both run on the LDS-ring kernel. Either way the rows are,
+    bit for bit, those of the same kernel over the resident layer."""
+    monkeypatch.setenv("R9K_STAGE_COLD", "1" if stage else "0")
+    E, H, I, topk, S, T = 8, 544, 160, 4, 4, 96
+    print(f"cached layer, 64-row blocks, stage={stage}", flush=True)
+    assert K.pick_mt(T * topk, E) == 4 and K.pick_moe_prefill_block(T * topk, E, H, I) is None
+    W13, W2 = make_w(dev, E, 2 * I, H, 81), make_w(dev, E, H, I, 82)
+    cache = C.LayerCache(0, C.to_host(W13.wq), C.to_host(W2.wq), W13.wsr, W2.wsr, 2 * I, H, H, I, S)
+    plain = R9700Mxfp4Experts.standalone(W13.wsr, W2.wsr)
+    cached = R9700Mxfp4Experts.standalone(cache.h_s13, cache.h_s2)
+    cached.r9k_cache = cache
+    monkeypatch.setattr(K, "DOWN_SUM_MAX_BYTES", 0)          # three launches on both sides
+    if not stage:
+        monkeypatch.setattr(K, "pick_mid_block", lambda *a: None)
+    seen, gemm = [], K.moe_gemm
+
+    def spy(a_q, a_s, w, *args, prefill=None, **kw):
+        seen.append((w.wq.device.type == "cpu", prefill))    # (over host memory, prefill cfg)
+        return gemm(a_q, a_s, w, *args, prefill=prefill, **kw)
+
+    g = torch.Generator().manual_seed(83)
+    for step in range(3):
+        x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+        logits = torch.randn(T, E, generator=g).to(torch.bfloat16).to(dev)
+        w, ids = K.moe_topk(logits, topk, True)
+        o0 = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
+        o1 = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
+        with monkeypatch.context() as m:
+            if not stage:
+                m.setattr(K, "MOE_PREFILL_CFG", -1)          # the decode kernel over the resident layer
+                m.setattr(K, "MOE_PREFILL_CFG_GATE_UP", -1)
+            plain.apply(o0, x, W13.wq, W2.wq, w, ids, "silu", E, None, None, None, None, None, None, False)
+        with monkeypatch.context() as m:
+            m.setattr(K, "moe_gemm", spy)
+            cached.apply(o1, x, cache.h_w13, cache.h_w2, w, ids, "silu", E, None, None, None, None, None, None, False)
+        torch.cuda.synchronize()
+        assert torch.equal(o0.view(torch.int16), o1.view(torch.int16)), f"step {step}"
+    assert len(seen) == 12 and all((cfg is None) == (not stage) for _, cfg in seen), seen
+    assert any(host for host, _ in seen) == (not stage)
+
+
+def test_host_offloaded_layer_keeps_the_decode_kernel(dev, monkeypatch):
+    """Experts whose weights lie in mapped host memory, without a cache: no LDS-ring launch at widths that would take
+    one (its ring re-reads bytes past the last step), and the resident layer's rows."""
+    E, H, I, topk, T = 8, 544, 160, 4, 96
+    W13, W2 = make_w(dev, E, 2 * I, H, 91), make_w(dev, E, H, I, 92)
+    h13, h2 = C.to_host(W13.wq), C.to_host(W2.wq)
+    layer = R9700Mxfp4Experts.standalone(W13.wsr, W2.wsr)
+    monkeypatch.setattr(K, "DOWN_SUM_MAX_BYTES", 0)
+    g = torch.Generator().manual_seed(93)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+    w, ids = K.moe_topk(torch.randn(T, E, generator=g).to(torch.bfloat16).to(dev), topk, True)
+    seen, gemm, outs = [], K.moe_gemm, []
+
+    def spy(*args, prefill=None, **kw):
+        seen.append(prefill)
+        return gemm(*args, prefill=prefill, **kw)
+
+    monkeypatch.setattr(K, "moe_gemm", spy)
+    for q13, q2 in ((W13.wq, W2.wq), (h13, h2)):
+        outs.append(torch.empty(T, H, dtype=torch.bfloat16, device=dev))
+        layer.apply(outs[-1], x, q13, q2, w, ids, "silu", E, None, None, None, None, None, None, False)
+    torch.cuda.synchronize()
+    assert seen == [K.MID_CFG, K.MID_CFG, None, None]
+    a, b = (o.float() for o in outs)                         # two kernels: fp32 sums in another order
+    assert float((a - b).norm() / a.norm()) <= 2e-3
+
+
 def test_stage_map_numbers_routed_cold_experts(dev):
     """r9k_lru_stage_map against a CPU restatement of its contract: the routed experts whose table entry is -1,
     numbered in ascending expert order (stage_map, the (expert, index) miss list, the count), capped at cap."""
