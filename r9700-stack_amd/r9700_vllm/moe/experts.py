@@ -198,7 +198,7 @@ class R9700Mxfp4Experts(_experts_base()):
         if M == 0:
             return
 
-        if M * bytes_per_token(topk, N1, K1, N2, K2) > BUF_LIMIT:
+        if M > 1 and M * bytes_per_token(topk, N1, K1, N2, K2) > BUF_LIMIT:
             for t0, t1 in chunk_tokens(M, topk, N1, K1, N2, K2):
                 self.apply(output[t0:t1], hidden_states[t0:t1], w1, w2, topk_weights[t0:t1], topk_ids[t0:t1],
                            activation, global_num_experts, expert_map, a1q_scale, a2_scale, workspace13, workspace2,

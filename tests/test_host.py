@@ -229,6 +229,30 @@ def test_tuned_table_lookup(tmp_path, monkeypatch):
     monkeypatch.setattr(tuned, "_TABLE", None)
 
 
+def test_apply_chunks_end_at_one_token(monkeypatch):
+    """A step past the buffer limit runs as its chunks, and a chunk of one token runs whatever its size."""
+    import r9700_vllm.moe.experts as X
+    layer = X.R9700Mxfp4Experts.standalone(torch.zeros(2, 3, 64, dtype=torch.uint8), torch.zeros(2, 2, 64, dtype=torch.uint8))
+    monkeypatch.setattr(X, "bytes_per_token", lambda *a: 1 << 32)
+    ran = []
+
+    class Reached(Exception):
+        pass
+
+    def first_step(numel, E):                                # what apply() does first for a step it does not split
+        ran.append(numel)
+        raise Reached
+
+    monkeypatch.setattr(K, "pick_mt", first_step)
+    x, w = torch.zeros(3, 64, dtype=torch.bfloat16), torch.zeros(2, 1)
+    step = lambda m: layer.apply(torch.zeros(m, 64), x[:m], w, w, torch.zeros(m, 2), torch.zeros(m, 2, dtype=torch.int32),
+                                 "silu", 2, None, None, None, None, None, None, False)
+    for m in (1, 3):
+        with pytest.raises(Reached):
+            step(m)
+    assert ran == [2, 2]                                     # one token of top-2 each time, no recursion on it
+
+
 def test_conversion_launch_rows():
     """One launch for tensors the conversion reads where they are; chunks for strided ones and for those elsewhere."""
     from r9700_vllm.quant.nvfp4 import _launch_rows
