@@ -521,20 +521,39 @@ def moe_gemm(a_q: torch.Tensor, a_s: torch.Tensor, w: Mxfp4Experts, out: torch.T
     return out
 
 
-# Dense MXFP4 linears on the 64- / 128-row LDS-ring kernel (r9k_moe_mid.hip, prefill cfgs MID_CFG / MID_CFG_BIG).
-# Below PREFILL_MIN_M rows it takes a step from DENSE_MID_M rows, earlier the more weight there is to stream per launch
-# (N * K): the decode kernel reads the activations once per wave, which costs little on a small weight. Measured on
-# MI355X, decode kernel (or r9k_dense_mxfp4_a8 up to 16 rows) -> this one, us: [17408, 5120] M = 4 / 6 / 16 / 32 / 48
-# 12.6 / 13.5 / 16.8 / 19.6 / 23.7 -> 12.9 / 12.8 / 12.8 / 13.3 / 14.8; [4096, 4096] M = 32 / 40 / 64 8.8 / 10.2 / 12.7
-# -> 10.4 / 9.8 / 9.7; [2048, 5120] M = 32 / 40 11.2 / 11.4 -> 11.0 / 10.5; [1024, 2048] M = 48 / 64 6.0 / 8.4 -> 7.1.
+# Dense MXFP4 linears on the 64- / 128-row LDS-ring kernel (r9k_moe_mid.hip, prefill cfgs MID_CFG / MID_CFG_BIG). Below
+# PREFILL_MIN_M rows it has to beat the decode kernel (r9k_dense_mxfp4_a8 up to 16 rows), whose waves are many where the
+# ring kernel's workgroups are few: one per 64 or 128 columns, each walking half of K. So it needs rows enough to share
+# the weights (the decode kernel pays for each 16 of them) or columns enough to fill the CUs. Measured on MI355X over 28
+# shapes with weights cold in every cache, decode kernel -> ring kernel, us:
+#   from 64 rows everywhere: [512, 512] 8.0 -> 4.7, [2048, 16384] 37.4 -> 30.2, [17408, 5120] 37.7 -> 20.1
+#   from 33 rows with N * K >= 2^23: [2048, 5120] 10.9 -> 10.1, [4096, 4096] 8.8 -> 8.9 (48 rows 9.2 -> 8.9), [8192, 8192]
+#     19.6 -> 17.3; not few columns by long K: [2048, 16384] 22 -> 28, [4096, 11008] 18.3 -> 21.0
+#   from 49 rows with less: [640, 2560] 8.7 -> 7.2, [2560, 320] 4.9 -> 4.8; not K of 9 to 16 K-tiles, which the decode
+#     kernel's four waves hold in one load batch each: [1024, 2048] 5.7 -> 6.6, [3072, 2048] 6.6 -> 6.8
+#   from 17 rows with N * K >= 2^25 and a third of the CUs busy (86 blocks of 128 columns): [11008, 4096] 12.6 -> 11.8,
+#     [17408, 5120] 19.7 -> 15.6; below that [8192, 8192] 14.5 -> 18.1, [5120, 17408] 26.1 -> 32.9
+#   from 12 rows with N * K >= 2^26 and one round of blocks: [17408, 5120] 15.0 -> 15.2 (16 rows 16.4 -> 15.6), [28672,
+#     8192] 29.7 -> 25.9; [16384, 2048] 5.9 -> 8.7, [34816, 5120] (272 blocks) 23.0 -> 27.2; 8 rows of [17408, 5120] 13.4 ->
+#     14.9
 MID_CFG, MID_CFG_BIG = 17, 10
-DENSE_MID_M = ((6, 1 << 25), (33, 1 << 23), (49, 0))           # (rows from, N * K from)
 _PREFILL_FORCED = "R9K_PREFILL_CFG" in os.environ or "R9K_PREFILL_CFG_SMALL" in os.environ
 
 
 def dense_mid_wanted(M: int, N: int, K: int) -> bool:
     """Whether a dense MXFP4 linear of M < PREFILL_MIN_M rows runs on the LDS-ring kernel's 64-row blocks."""
-    return N % 16 == 0 and K % GROUP == 0 and any(M >= m and N * K >= nk for m, nk in DENSE_MID_M)
+    if M < 12 or N % 16 or K % GROUP:
+        return False
+    if M >= 64:
+        return True
+    nk, blocks, ktiles = N * K, -(-N // 128), -(-K // 128)
+    if M >= 33:
+        if nk >= 1 << 23:
+            return ktiles <= 64 or blocks >= 40
+        return M >= 49 and not 8 < ktiles <= 16
+    if M >= 17:
+        return nk >= 1 << 25 and blocks >= 86
+    return nk >= 1 << 26 and 86 <= blocks <= 256
 
 
 def dense_prefill_cfg(M: int, N: int, K: int) -> int:
