@@ -662,30 +662,44 @@ DEVICE_BLOCKS_MIN = int(os.environ.get("R9K_MOE_DEVICE_BLOCKS_MIN", "1024"))
 DEVICE_MIN_ROWS = int(os.environ.get("R9K_MOE_DEVICE_MIN_ROWS", "22"))
 
 
-# Routed steps of small experts (gate_up codes below SPLIT_DECODE_MIN_BYTES) from MID_MIN_ROWS rows an expert run on
-# 64-row blocks of the LDS-ring kernel, from MID_BIG_ROWS on 256-row blocks (128-row ones where a K is not a multiple of
-# 128), all without splitting the tables: a 64-row block streams its expert's weights once, so experts with a handful
-# of rows cost little more than their weights. Measured on MI355X, whole layer, us: 288 experts, hidden 2048, intermediate
-# 512, T = 600 / 1024 / 2048 / 4096: 206 / 222 / 225 / 273 on split tables, 189 / 189 / 202 / 250 on 256-row blocks, 183 /
-# 158 / 191 / 287 on 64-row ones (under Zipf(1.1) routing 139 / 140 / 183 / 253, 150 / 138 / 178 / 250 and 142 / 123 / 172
-# / 267); 512 experts, top-10, hidden 2560, intermediate 320 (GEMMs alone): T = 500 / 1000 / 1600 decode blocks 165 / 217 /
-# 299, 64-row blocks 155 / 163 / 176; T = 4096 (80 rows an expert) 64-row 307, 128-row 243.
-MID_MIN_ROWS, MID_BIG_ROWS = 10, 64
+# Routed steps of small experts (gate_up codes below SPLIT_DECODE_MIN_BYTES) run on 64-row blocks of the LDS-ring kernel
+# from MID_MIN_ROWS rows an expert: a 64-row block streams its expert's weights once, so experts with a handful of rows
+# cost little more than their weights. Measured on MI355X over 23 layers (0.2 to 3.9 MB of gate_up codes an expert, 16 to
+# 512 experts) under uniform, Zipf(0.6) and Zipf(1.1) routing, whole layer, old -> new: geometric mean 0.81 at 10 rows,
+# 0.78 at 48. A down product whose K fills its 128-wide tiles by three quarters or less (K = 160, 192) starts at
+# MID_MIN_ROWS + 2: 128 experts, hidden 4096, intermediate 192 at 10 / 12 rows 68.8 -> 74.3, 74.8 -> 74.1 us.
+# Where a K is not a multiple of 128, 128-row blocks follow from MID_ODD_ROWS: 512 experts, hidden 2560, intermediate 320
+# at 64 / 72 / 96 rows 0.485 / 0.438 / 0.423 of the decode blocks' time against 0.499 / 0.485 / 0.466 on 64-row blocks
+# (skewed 0.52 against 0.50). Else, from MID_BIG_ROWS, the 256-row blocks without split tables, whose two more launches a
+# GEMM cost more than they save while the layer is small: 288 experts, hidden 2048, intermediate 512, uniform / Zipf(0.6) /
+# Zipf(1.1), us: 72 rows 243 / 260 / 193 split, 225 / 224 / 189 on 64-row blocks, 225 / 272 / 204 on 256-row ones; 96 rows
+# 264 / 284 / 228, 248 / 253 / 230 and 243 / 294 / 224. A layer of MID_SPLIT_BYTES gate_up codes and more keeps its split
+# tables, from MID_SPLIT_ROWS: 256 experts, hidden 3072, intermediate 1024 on 256-row blocks 0.96 / 1.09 / 1.14 of the
+# split tables' time at 80 rows, 0.96 / 1.06 / 1.09 at 128 (512 experts, hidden 2048, intermediate 1024 at 72 0.98 / 1.19 /
+# 1.10); on 64-row blocks 0.96 / 0.95 / 1.03 at 64 rows, 1.06 / 0.97 / 1.05 at 80.
+MID_MIN_ROWS, MID_BIG_ROWS, MID_ODD_ROWS, MID_SPLIT_ROWS = 10, 80, 64, 72
+MID_SPLIT_BYTES = 512 << 20
 
 
 def pick_mid_block(numel: int, num_experts: int, K1: int, K2: int):
     """(cfg, rows per routing block) for a routed MXFP4 step on the LDS-ring kernel, else None."""
     per = numel / max(1, min(num_experts, numel))
-    if per < MID_MIN_ROWS or not small_experts(K1, K2):
+    if not small_experts(K1, K2) or per < MID_MIN_ROWS + (2 if 4 * K2 <= 3 * (-(-K2 // 128) * 128) else 0):
         return None
-    if per < MID_BIG_ROWS:
+    odd = K1 % 128 or K2 % 128
+    if per < (MID_ODD_ROWS if odd else MID_BIG_ROWS if unsplit_layer(num_experts, K1, K2) else MID_SPLIT_ROWS):
         return MID_CFG, prefill_block(MID_CFG)
-    return (MID_CFG_BIG, prefill_block(MID_CFG_BIG)) if K1 % 128 or K2 % 128 else None
+    return (MID_CFG_BIG, prefill_block(MID_CFG_BIG)) if odd else None
 
 
 def small_experts(K1: int, K2: int) -> bool:
     """Experts with fewer than SPLIT_DECODE_MIN_BYTES of gate_up codes (K1 * 2 K2 / 2 bytes)."""
     return K1 * K2 < SPLIT_DECODE_MIN_BYTES
+
+
+def unsplit_layer(num_experts: int, K1: int, K2: int) -> bool:
+    """Layers of small experts whose prefill steps run on 256-row blocks without split tables."""
+    return small_experts(K1, K2) and num_experts * K1 * K2 < MID_SPLIT_BYTES
 
 
 def big_block_cfg(K1: int, K2: int):

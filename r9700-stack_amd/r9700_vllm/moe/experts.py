@@ -271,7 +271,7 @@ class R9700Mxfp4Experts(_experts_base()):
             if mid is not None and route.take(layer, topk_ids, blk, numel) is not None:
                 mid = None
             split = (plain and mid is None and K.split_wanted(numel, E, K1, K2)
-                     and (host or not (big is not None and K.small_experts(K1, K2))))
+                     and (host or not (big is not None and K.unsplit_layer(E, K1, K2))))
             if mid is not None:
                 pf_gate = pf_down = mid[0]
                 blk = mid[1]
