@@ -540,9 +540,24 @@ MID_CFG, MID_CFG_BIG = 17, 10
 _PREFILL_FORCED = "R9K_PREFILL_CFG" in os.environ or "R9K_PREFILL_CFG_SMALL" in os.environ
 
 
+def _on(env, name: str, overrides) -> bool:
+    """Switch `name`: on unless it is set to another value than 1 or, where it is not set, one of `overrides` is -- the
+    variables that chose these calls' kernel before there was another one, and still do."""
+    return env.get(name, "0" if any(v in env for v in overrides) else "1") == "1"
+
+
+def _dense_mid_on(env) -> bool:
+    own_table = env.get("R9K_TUNED", "0") not in ("", "0")
+    return _on(env, "R9K_DENSE_MID", ("R9K_DENSE_A8_MAX_M",) + (("R9K_TUNED",) if own_table else ()))
+
+
+DENSE_MID = _dense_mid_on(os.environ)
+
+
 def dense_mid_wanted(M: int, N: int, K: int) -> bool:
-    """Whether a dense MXFP4 linear of M < PREFILL_MIN_M rows runs on the LDS-ring kernel's 64-row blocks."""
-    if M < 12 or N % 16 or K % GROUP:
+    """Whether a dense MXFP4 linear of M < PREFILL_MIN_M rows runs on the LDS-ring kernel's 64-row blocks.
+    R9K_DENSE_MID=0, a launch table of one's own (R9K_TUNED) or R9K_DENSE_A8_MAX_M keep it off."""
+    if not DENSE_MID or M < 12 or N % 16 or K % GROUP:
         return False
     if M >= 64:
         return True
@@ -662,7 +677,7 @@ DEVICE_BLOCKS_MIN = int(os.environ.get("R9K_MOE_DEVICE_BLOCKS_MIN", "1024"))
 DEVICE_MIN_ROWS = int(os.environ.get("R9K_MOE_DEVICE_MIN_ROWS", "22"))
 
 
-# Routed steps of small experts (gate_up codes below SPLIT_DECODE_MIN_BYTES) run on 64-row blocks of the LDS-ring kernel
+# Routed steps of small experts (gate_up codes below MID_MAX_BYTES) run on 64-row blocks of the LDS-ring kernel
 # from MID_MIN_ROWS rows an expert: a 64-row block streams its expert's weights once, so experts with a handful of rows
 # cost little more than their weights. Measured on MI355X over 23 layers (0.2 to 3.9 MB of gate_up codes an expert, 16 to
 # 512 experts) under uniform, Zipf(0.6) and Zipf(1.1) routing, whole layer, old -> new: geometric mean 0.81 at 10 rows,
@@ -677,8 +692,15 @@ DEVICE_MIN_ROWS = int(os.environ.get("R9K_MOE_DEVICE_MIN_ROWS", "22"))
 # tables, from MID_SPLIT_ROWS: 256 experts, hidden 3072, intermediate 1024 on 256-row blocks 0.96 / 1.09 / 1.14 of the
 # split tables' time at 80 rows, 0.96 / 1.06 / 1.09 at 128 (512 experts, hidden 2048, intermediate 1024 at 72 0.98 / 1.19 /
 # 1.10); on 64-row blocks 0.96 / 0.95 / 1.03 at 64 rows, 1.06 / 0.97 / 1.05 at 80.
-MID_MIN_ROWS, MID_BIG_ROWS, MID_ODD_ROWS, MID_SPLIT_ROWS = 10, 80, 64, 72
-MID_SPLIT_BYTES = 512 << 20
+# R9K_MOE_MID=0 turns all of it off, and so does setting a variable that chooses these steps' blocks itself.
+MID = _on(os.environ, "R9K_MOE_MID", ("R9K_MOE_MT", "R9K_MOE_PREFILL_CFG", "R9K_MOE_PREFILL_CFG1", "R9K_MOE_PREFILL_CFG_BIG",
+                                      "R9K_PREFILL_MOE_ROWS"))
+MID_MIN_ROWS = int(os.environ.get("R9K_MOE_MID_MIN_ROWS", "10"))
+MID_BIG_ROWS = int(os.environ.get("R9K_MOE_MID_BIG_ROWS", "80"))
+MID_ODD_ROWS = int(os.environ.get("R9K_MOE_MID_ODD_ROWS", "64"))
+MID_SPLIT_ROWS = int(os.environ.get("R9K_MOE_MID_SPLIT_ROWS", "72"))
+MID_MAX_BYTES = int(os.environ.get("R9K_MOE_MID_MAX_BYTES", str(4 << 20)))
+MID_SPLIT_BYTES = int(os.environ.get("R9K_MOE_MID_SPLIT_BYTES", str(512 << 20)))
 
 
 def pick_mid_block(numel: int, num_experts: int, K1: int, K2: int):
@@ -693,8 +715,9 @@ def pick_mid_block(numel: int, num_experts: int, K1: int, K2: int):
 
 
 def small_experts(K1: int, K2: int) -> bool:
-    """Experts with fewer than SPLIT_DECODE_MIN_BYTES of gate_up codes (K1 * 2 K2 / 2 bytes)."""
-    return K1 * K2 < SPLIT_DECODE_MIN_BYTES
+    """Experts with fewer than MID_MAX_BYTES of gate_up codes (K1 * 2 K2 / 2 bytes), and too few for split tables at decode
+    widths (a lower SPLIT_DECODE_MIN_BYTES hands them to those)."""
+    return MID and K1 * K2 < min(MID_MAX_BYTES, SPLIT_DECODE_MIN_BYTES)
 
 
 def unsplit_layer(num_experts: int, K1: int, K2: int) -> bool:
