@@ -25,9 +25,15 @@ _registered = False
 class IdentityTables:
     """Routing tables that make the grouped GEMM a dense one: rows 0..Mpad-1 in order, every block on expert 0,
     Mpad = M rounded up to the block. Built once per (device, Mpad, block) and reused (graph capture needs fixed
-    addresses, and a decode step asks for the same few shapes every time)."""
+    addresses, and a decode step asks for the same few shapes every time). A width first met under capture gets tables
+    that the graph fills itself: device fills only, and not kept, since they hold nothing before the first replay."""
 
     _cache: dict = {}
+
+    @staticmethod
+    def _build(device: torch.device, mpad: int, block: int):
+        i32 = dict(dtype=torch.int32, device=device)
+        return torch.arange(mpad, **i32), torch.full((mpad // block,), 0, **i32), torch.full((1,), mpad, **i32)
 
     @classmethod
     def get(cls, device: torch.device, M: int, block: int):
@@ -35,9 +41,9 @@ class IdentityTables:
         key = (device.type, device.index, mpad, block)
         t = cls._cache.get(key)
         if t is None:
-            i32 = dict(dtype=torch.int32, device=device)
-            t = cls._cache[key] = (torch.arange(mpad, **i32), torch.zeros(mpad // block, **i32),
-                                   torch.tensor([mpad], **i32))
+            t = cls._build(device, mpad, block)
+            if not (device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
+                cls._cache[key] = t
         return t
 
 
