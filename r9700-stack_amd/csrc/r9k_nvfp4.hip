@@ -338,6 +338,58 @@ __global__ void __launch_bounds__(256) nvfp4_to_mxfp4_kernel(const uint8_t* __re
   out_e[b] = (uint8_t)eb;
 }
 
+// (E2M1[c] * s) / rd for the 16 codes of one group, with IEEE division semantics, from two divisions: every E2M1
+// magnitude is 2^j or 1.5 * 2^j, and scaling a correctly rounded quotient by 2^j is exact while it stays normal, so
+// RN(1.5^b * 2^j * s / rd) = 2^j * RN(1.5^b * s / rd). Groups whose quotients could leave the normal range (or a
+// non-finite / non-positive divisor) divide per element.
+__device__ __forceinline__ void dequant_group(const uint32_t w0, const uint32_t w1, float s, float rd, float* x) {
+  const float q1 = s / rd, q3 = (1.5f * s) / rd;
+  const float aq1 = fabsf(q1), aq3 = fabsf(q3);
+  const bool fast = (aq1 >= 0x1p-125f || aq1 == 0.f) && aq3 <= 0x1p125f && rd > 0.f && rd <= 3.0e38f;
+  float v[16];
+  e2m1_decode8(w0, *reinterpret_cast<float(*)[8]>(v));
+  e2m1_decode8(w1, *reinterpret_cast<float(*)[8]>(v + 8));
+  if (fast) {
+    // V = E2M1[c] = +-2^j (mantissa bit clear) or +-1.5 * 2^j (set): x = (V with its mantissa cleared) * (q1 or q3)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const uint32_t vb = __float_as_uint(v[i]);
+      x[i] = __uint_as_float(vb & 0xff800000u) * ((vb & 0x00400000u) ? q3 : q1);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; i++) x[i] = (v[i] * s) / rd;
+  }
+}
+
+// The conversion of weights too small to fill the chip, element by element (search_block on the block's values): there
+// a launch takes as long as its longest wave, and a wave with one block for search_nvfp4_block_exact takes that serial
+// path's ~10 us. Blocks, this kernel -> the other, us: 8192 (512 x 512) 6.9 -> 12.0, 65536 (1024 x 2048) 7.0 -> 13-17,
+// 2^19 (4096 x 4096) 20.4-23.0 -> 19.2-21.3 (22.6 -> 27.6 at divisor 1, whose candidates often tie), 2.8M (17408 x 5120)
+// 85-93 -> 47-62. Same codes and bytes.
+constexpr long SMALL_BLOCKS = 1L << 19;
+
+__global__ void __launch_bounds__(256) nvfp4_to_mxfp4_small_kernel(const uint8_t* __restrict__ packed,
+                                                                   const uint8_t* __restrict__ s16,
+                                                                   const float* __restrict__ row_div,
+                                                                   uint8_t* __restrict__ out_p,
+                                                                   uint8_t* __restrict__ out_e, uint32_t nblk,
+                                                                   DivMagic bpr) {
+  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nblk) return;
+  const uint4 pk = *reinterpret_cast<const uint4*>(packed + (size_t)b * 16);
+  const uint32_t sc = *reinterpret_cast<const uint16_t*>(s16 + (size_t)b * 2);
+  const float rd = row_div[div_by(b, bpr)];
+  const float s0 = e4m3_to_f32(sc & 0xffu), s1 = e4m3_to_f32(sc >> 8);
+  float x[32];
+  dequant_group(pk.x, pk.y, s0, rd, x);
+  dequant_group(pk.z, pk.w, s1, rd, x + 16);
+  uint32_t bw[4];
+  const uint32_t eb = search_block(x, bw);
+  *reinterpret_cast<uint4*>(out_p + (size_t)b * 16) = make_uint4(bw[0], bw[1], bw[2], bw[3]);
+  out_e[b] = (uint8_t)eb;
+}
+
 // fp32 weights [N, K] (row stride ld floats) -> MXFP4 by the same search (quantize_mxfp4_search on any weight).
 __global__ void __launch_bounds__(256) mxfp4_search_kernel(const float* __restrict__ w, long ld,
                                                            uint8_t* __restrict__ out_p, uint8_t* __restrict__ out_e,
@@ -374,7 +426,8 @@ extern "C" int r9k_nvfp4_to_mxfp4(long packed, long s16, long row_div, long out_
   const long step = std::max(1L, 0x7fffff00L / bpr);
   for (long r0 = 0; r0 < N; r0 += step) {
     const long n = std::min(step, N - r0) * bpr, b0 = r0 * bpr;
-    hipLaunchKernelGGL(nvfp4_to_mxfp4_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(n <= SMALL_BLOCKS ? nvfp4_to_mxfp4_small_kernel : nvfp4_to_mxfp4_kernel,
+                       dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                        (const uint8_t*)packed + b0 * 16, (const uint8_t*)s16 + b0 * 2, (const float*)row_div + r0,
                        (uint8_t*)out_packed + b0 * 16, (uint8_t*)out_e8m0 + b0, (uint32_t)n, div_magic((uint32_t)bpr));
     if (hipGetLastError() != hipSuccess) return -6;

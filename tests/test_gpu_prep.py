@@ -62,10 +62,9 @@ def test_nvfp4_conversion_of_strided_tensors_stays_chunked(dev):
     assert extra <= outputs + 3 * chunk + (1 << 20), (extra, outputs, chunk)      # two chunks may be alive, and their rounding
 
 
-@pytest.mark.parametrize("rd", [1.0, 448.0, 2688.0 / 3.7, 1e30, 1e-30, 3.3e38])
-def test_nvfp4_search_branches(dev, rd):
-    """Uniform blocks, every scale byte (zero, subnormal, negative, NaN), one-magnitude and all-zero blocks, groups whose
-    scales lie far apart, exact ties of the two candidates, divisors that leave the exact quotients' range."""
+def search_blocks(rd):
+    """Checkpoint tensors of 256 x 512: uniform blocks, every scale byte (zero, subnormal, negative, NaN), one-magnitude
+    and all-zero blocks, groups whose scales lie far apart, exact ties of the two candidates."""
     g = torch.Generator().manual_seed(int(abs(np.log(rd)) * 10) + 1)
     N, Kd = 256, 512
     packed = torch.randint(0, 256, (N, Kd // 2), generator=g, dtype=torch.int32).to(torch.uint8)
@@ -78,9 +77,33 @@ def test_nvfp4_search_branches(dev, rd):
     s16[72:80] = torch.tensor([1, 0x7e], dtype=torch.uint8).repeat(16)      # smallest and largest scale in one block
     s16[80:128] = (s16[80:128] & 0x78) | 0x08                               # power-of-two scales: exact values, ties
     s16[128:144, 0::2] = 0                                                  # one group of a block all zero
-    div = torch.full((N,), rd)
+    return packed, s16, torch.full((N,), rd)
+
+
+DIVISORS = [1.0, 448.0, 2688.0 / 3.7, 1e30, 1e-30, 3.3e38]                  # some leave the exact quotients' range
+
+
+@pytest.mark.parametrize("rd", DIVISORS)
+def test_nvfp4_search_branches(dev, rd):
+    """The conversion of a small weight (element by element) on blocks that reach each branch of the search."""
+    packed, s16, div = search_blocks(rd)
     pm, em = NV.nvfp4_to_mxfp4(packed.to(dev), s16.view(torch.float8_e4m3fn).to(dev), div.to(dev))
     po, eo = O.nvfp4_to_mxfp4(packed.numpy(), s16.numpy(), div.numpy())
     bad = np.argwhere(em.cpu().numpy() != eo)
     assert bad.size == 0, f"exponents differ at {bad[:4].tolist()}"
     assert np.array_equal(pm.cpu().numpy(), po)
+
+
+@pytest.mark.parametrize("rd", DIVISORS)
+def test_nvfp4_search_by_magnitudes(dev, rd):
+    """The same blocks often enough for the kernel of large weights (more than 2^19 blocks; three rows short of whole
+    copies, so the last workgroup is partly idle): every row has the oracle's codes and exponents."""
+    packed, s16, div = search_blocks(rd)
+    po, eo = O.nvfp4_to_mxfp4(packed.numpy(), s16.numpy(), div.numpy())
+    n, rows = 129, 129 * 256 - 3
+    assert rows * 16 > 1 << 19 and rows * 16 % 256
+    many = lambda t: t.to(dev).repeat(n, *[1] * (t.dim() - 1))[:rows].contiguous()
+    pm, em = NV.nvfp4_to_mxfp4(many(packed), many(s16).view(torch.float8_e4m3fn), many(div))
+    bad = (em != many(torch.from_numpy(eo))).nonzero()
+    assert bad.numel() == 0, f"exponents differ at {bad[:4].tolist()}"
+    assert torch.equal(pm, many(torch.from_numpy(po)))
