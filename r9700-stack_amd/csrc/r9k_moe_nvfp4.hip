@@ -315,6 +315,7 @@ struct PvStage {
 struct PvW { u32x4 k[4]; };           // a column tile's widened weights of one K-tile
 constexpr size_t PV_SMEM = PV_NS * sizeof(PvStage) + PV_BM * (sizeof(int) + 2 * sizeof(float));
 
+template <bool PIPE>
 __global__ void __launch_bounds__(PV_THREADS, 2) nvfp4_prefill_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint8_t* __restrict__ Ws, const float* __restrict__ Wg, uint16_t* __restrict__ C,
@@ -400,92 +401,133 @@ __global__ void __launch_bounds__(PV_THREADS, 2) nvfp4_prefill_kernel(
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-  // Ahead of the loop: K-tiles 0 and 1 of everything and 2 of the weights on their way, K-tile 0's weights widened, the
-  // raw weights of K-tile 1's first two column tiles and the raw activations of row tile 1 in registers
-  issue_a(0, 0);
-  issue_w(0, 0);
-  issue_w(1, SL);
-  issue_a(1, SL);
-  issue_w(2, 2 * SL);
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(PV_DMA) : "memory");
-  PvW B[2][3], b3;                                             // column tile 3 is widened in place
-  u32x4 a[4], rl = ld_lo(0, 0), rh = ld_hi(0, 0), rw[2];
-  uint32_t rs;
-  h2 gs;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    rw[1] = ld_w(0, j);
-    gs = scales_f16(ld_s(0, j));
-    PvW& d = j < 3 ? B[0][j] : b3;
-#pragma unroll
-    for (int t = 0; t < 4; t++) d.k[t] = __builtin_bit_cast(u32x4, e2m1x8_f16(rw[1][t], gs[t >> 1]));
-  }
-  a[0] = __builtin_bit_cast(u32x4, e4m3x8_f16(rl.x, rl.y));
-  a[1] = __builtin_bit_cast(u32x4, e4m3x8_f16(rl.z, rl.w));
-  a[2] = __builtin_bit_cast(u32x4, e4m3x8_f16(rh.x, rh.y));
-  a[3] = __builtin_bit_cast(u32x4, e4m3x8_f16(rh.z, rh.w));
-  rl = ld_lo(0, 1);
-  rw[0] = ld_w(SL, 0);
-  rs = ld_s(SL, 0);
-  __builtin_amdgcn_s_waitcnt(0xC07F);                          // K-tile 0's weights are read: slot 0 takes K-tile 3's
-  asm volatile("s_barrier" ::: "memory");
-  issue_a(2, 2 * SL);
-  issue_w(3, 0);
-
-  // One K-tile kt (slot c0; c1, c2 hold kt + 1, kt + 2) from the widened weights bc and b3. Row tile i's 16 MFMAs run
-  // step by step (p / 4) over the 4 column tiles, and each carries one conversion pair of row tile i + 1's activations
-  // and one of the next K-tile's column tile i, four MFMAs behind, so that activations and column tile 3 replace their
-  // predecessors in the same registers right after their last use (step 3 of each in the next row tile's first four).
-  // In row tile 2 a barrier publishes the activations of kt + 1 and the weights of kt + 2 (issued a K-tile ago; the 7
-  // loads after them stay in flight); every wave has read the activations of kt and the weights of kt + 1 by then, so
-  // their slots take those of kt + 3 and kt + 4.
-  auto step = [&](int kt, uint32_t c0, uint32_t c1, uint32_t c2, PvW (&bc)[3], PvW (&bn)[3]) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-#pragma unroll
-      for (int p = 0; p < 16; p++) {
-        if (i == 2 && p == 8) {
-          __builtin_amdgcn_s_waitcnt(0xC07F);
-          asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(PV_DMA) : "memory");
-          issue_a(kt + 3, c0);
-          issue_w(kt + 4, c1);
-        }
-        const int t = p >> 2, j = p & 3;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            __builtin_bit_cast(h8, a[t]), __builtin_bit_cast(h8, (j < 3 ? bc[j] : b3).k[t]), acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (p == 4) {
-          gs = scales_f16(rs);
-          rh = i < 3 ? ld_hi(c0, i + 1) : ld_hi(c1, 0);
-          rw[(i + 1) & 1] = i < 3 ? ld_w(c1, i + 1) : ld_w(c2, 0);
-          rs = i < 3 ? ld_s(c1, i + 1) : ld_s(c2, 0);
-        }
-        if (p == 12) rl = i < 2 ? ld_lo(c0, i + 2) : ld_lo(c1, i - 2);
-        const int u = p >= 4 ? t - 1 : 3;                      // the step converted here
-        const int jc = p >= 4 ? i : (i + 3) & 3;               // and its column tile (i == 0: of this K-tile)
-        const uint32_t av = u < 2 ? rl[2 * u + (j >> 1)] : rh[2 * u + (j >> 1) - 4];
-        const h2 pa = j & 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)av, 1.0f, true)
-                            : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)av, 1.0f, false);
-        a[u][j] = __builtin_bit_cast(uint32_t, pa);
-        const h2 pw = e2m1x2_f16(rw[jc & 1][u], j) * (h2){gs[u >> 1], gs[u >> 1]};
-        (jc < 3 ? bn[jc] : b3).k[u][j] = __builtin_bit_cast(uint32_t, pw);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+  if constexpr (PIPE) {
+    // Ahead of the loop: K-tiles 0 and 1 of everything and 2 of the weights on their way, K-tile 0's weights widened, the
+    // raw weights of K-tile 1's first two column tiles and the raw activations of row tile 1 in registers
+    issue_a(0, 0);
+    issue_w(0, 0);
+    issue_w(1, SL);
+    issue_a(1, SL);
+    issue_w(2, 2 * SL);
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(PV_DMA) : "memory");
+    PvW B[2][3], b3;                                             // column tile 3 is widened in place
+    u32x4 a[4], rl = ld_lo(0, 0), rh = ld_hi(0, 0), rw[2];
+    uint32_t rs;
+    h2 gs;
+  #pragma unroll
+    for (int j = 0; j < 4; j++) {
+      rw[1] = ld_w(0, j);
+      gs = scales_f16(ld_s(0, j));
+      PvW& d = j < 3 ? B[0][j] : b3;
+  #pragma unroll
+      for (int t = 0; t < 4; t++) d.k[t] = __builtin_bit_cast(u32x4, e2m1x8_f16(rw[1][t], gs[t >> 1]));
     }
-  };
-  uint32_t c0 = 0, c1 = SL, c2 = 2 * SL;
-  int kt = 0;
-  for (; kt + 1 < nkt; kt += 2) {
-    step(kt, c0, c1, c2, B[0], B[1]);
-    step(kt + 1, c1, c2, c0, B[1], B[0]);
-    const uint32_t x = c0;
-    c0 = c2;
-    c2 = c1;
-    c1 = x;
+    a[0] = __builtin_bit_cast(u32x4, e4m3x8_f16(rl.x, rl.y));
+    a[1] = __builtin_bit_cast(u32x4, e4m3x8_f16(rl.z, rl.w));
+    a[2] = __builtin_bit_cast(u32x4, e4m3x8_f16(rh.x, rh.y));
+    a[3] = __builtin_bit_cast(u32x4, e4m3x8_f16(rh.z, rh.w));
+    rl = ld_lo(0, 1);
+    rw[0] = ld_w(SL, 0);
+    rs = ld_s(SL, 0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);                          // K-tile 0's weights are read: slot 0 takes K-tile 3's
+    asm volatile("s_barrier" ::: "memory");
+    issue_a(2, 2 * SL);
+    issue_w(3, 0);
+
+    // One K-tile kt (slot c0; c1, c2 hold kt + 1, kt + 2) from the widened weights bc and b3. Row tile i's 16 MFMAs run
+    // step by step (p / 4) over the 4 column tiles, and each carries one conversion pair of row tile i + 1's activations
+    // and one of the next K-tile's column tile i, four MFMAs behind, so that activations and column tile 3 replace their
+    // predecessors in the same registers right after their last use (step 3 of each in the next row tile's first four).
+    // In row tile 2 a barrier publishes the activations of kt + 1 and the weights of kt + 2 (issued a K-tile ago; the 7
+    // loads after them stay in flight); every wave has read the activations of kt and the weights of kt + 1 by then, so
+    // their slots take those of kt + 3 and kt + 4.
+    auto step = [&](int kt, uint32_t c0, uint32_t c1, uint32_t c2, PvW (&bc)[3], PvW (&bn)[3]) {
+  #pragma unroll
+      for (int i = 0; i < 4; i++) {
+  #pragma unroll
+        for (int p = 0; p < 16; p++) {
+          if (i == 2 && p == 8) {
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(PV_DMA) : "memory");
+            issue_a(kt + 3, c0);
+            issue_w(kt + 4, c1);
+          }
+          const int t = p >> 2, j = p & 3;
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(h8, a[t]), __builtin_bit_cast(h8, (j < 3 ? bc[j] : b3).k[t]), acc[i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (p == 4) {
+            gs = scales_f16(rs);
+            rh = i < 3 ? ld_hi(c0, i + 1) : ld_hi(c1, 0);
+            rw[(i + 1) & 1] = i < 3 ? ld_w(c1, i + 1) : ld_w(c2, 0);
+            rs = i < 3 ? ld_s(c1, i + 1) : ld_s(c2, 0);
+          }
+          if (p == 12) rl = i < 2 ? ld_lo(c0, i + 2) : ld_lo(c1, i - 2);
+          const int u = p >= 4 ? t - 1 : 3;                      // the step converted here
+          const int jc = p >= 4 ? i : (i + 3) & 3;               // and its column tile (i == 0: of this K-tile)
+          const uint32_t av = u < 2 ? rl[2 * u + (j >> 1)] : rh[2 * u + (j >> 1) - 4];
+          const h2 pa = j & 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)av, 1.0f, true)
+                              : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)av, 1.0f, false);
+          a[u][j] = __builtin_bit_cast(uint32_t, pa);
+          const h2 pw = e2m1x2_f16(rw[jc & 1][u], j) * (h2){gs[u >> 1], gs[u >> 1]};
+          (jc < 3 ? bn[jc] : b3).k[u][j] = __builtin_bit_cast(uint32_t, pw);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    uint32_t c0 = 0, c1 = SL, c2 = 2 * SL;
+    int kt = 0;
+    for (; kt + 1 < nkt; kt += 2) {
+      step(kt, c0, c1, c2, B[0], B[1]);
+      step(kt + 1, c1, c2, c0, B[1], B[0]);
+      const uint32_t x = c0;
+      c0 = c2;
+      c2 = c1;
+      c1 = x;
+    }
+    if (kt < nkt) step(kt, c0, c1, c2, B[0], B[1]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // no DMA may outlive the workgroup's LDS
+  } else {
+    // few K-tiles: two ahead in the ring, each widened ahead of its MFMAs, nothing loaded past the last
+    issue_a(0, 0);
+    issue_w(0, 0);
+    if (nkt > 1) {
+      issue_a(1, SL);
+      issue_w(1, SL);
+    }
+    uint32_t sl = 0;
+    for (int kt = 0; kt < nkt; kt++) {
+      if (kt + 1 < nkt) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(PV_DMA) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (kt + 2 < nkt) {                                      // into the slot read in the iteration before
+        const uint32_t s2 = sl == 0 ? 2 * SL : sl - SL;
+        issue_a(kt + 2, s2);
+        issue_w(kt + 2, s2);
+      }
+      h8 b[4][4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const u32x4 bw = ld_w(sl, j);
+        const h2 gs = scales_f16(ld_s(sl, j));
+#pragma unroll
+        for (int t = 0; t < 4; t++) b[j][t] = e2m1x8_f16(bw[t], gs[t >> 1]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const u32x4 lo = ld_lo(sl, i), hi = ld_hi(sl, i);
+        const h8 a[4] = {e4m3x8_f16(lo.x, lo.y), e4m3x8_f16(lo.z, lo.w), e4m3x8_f16(hi.x, hi.y),
+                         e4m3x8_f16(hi.z, hi.w)};
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int t = 0; t < 4; t++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], b[j][t], acc[i][j], 0, 0, 0);
+      }
+      sl = sl == 2 * SL ? 0 : sl + SL;
+    }
   }
-  if (kt < nkt) step(kt, c0, c1, c2, B[0], B[1]);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // no DMA may outlive the workgroup's LDS
 
   // epilogue: lane holds column c of each column tile, rows 4g .. 4g + 3 of each row tile; out = bf16(v * ((Wg[n] *
   // As[row]) * topk_w[row])), the row factors from LDS and the lane's 4 column multipliers loaded together. Branch-free:
@@ -708,13 +750,24 @@ int r9k_nvfp4_prefill_launch(long a, long as, long wq, long ws, long wg, long c,
   // the DMA addresses activations and one expert's codes through 32-bit offsets
   if ((long)((numel + a_row_div - 1) / a_row_div) * K >= (1L << 32) || wq_estride >= (1L << 32)) return -3;
   if ((long)numel * N * 2 >= (1L << 31)) return -3;             // the epilogue's raw output buffer
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(nvfp4_prefill_kernel),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)PV_SMEM);
-  if (attr != hipSuccess) return -6;
-  hipLaunchKernelGGL(nvfp4_prefill_kernel, grid, dim3(PV_THREADS), PV_SMEM, (hipStream_t)stream, (const uint8_t*)a,
-                     (const float*)as, (const uint8_t*)wq, (const uint8_t*)ws, (const float*)wg, (uint16_t*)c,
-                     (const int*)sorted_ids, (const int*)expert_ids, (const int*)ntpp, (const float*)topk_w,
-                     wq_estride, ws_estride, wg_estride, numel, a_row_div, K, N, blk, subs);
+  // The software pipeline loads three K-tiles past the last and pays a prologue. Up to two K-tiles that costs more than
+  // it hides ([16384, 256] at 128 / 1024 / 4096 rows 7.50 / 19.6 / 60.9 us plain, 7.65 / 20.9 / 65.9 pipelined), and up to
+  // four where the tiles fill the chip twice over, whose other workgroups hide the widening (512 K: [16384] at 4096 rows
+  // 85.6 / 87.5, 288 experts x 2048 at 128 rows each 161 / 170; with fewer tiles [4096] at 1024 rows 10.7 / 10.4). From
+  // five on the pipeline wins or is even up to ~100M outputs ([4096, 1024] at 1024 rows 15.3 / 14.4).
+  const int nkt = (K + NV_KT - 1) / NV_KT;
+  const bool pipe = nkt > 4 || (nkt > 2 && (long)grid.x * ny < 1024);
+  static const hipError_t attr[2] = {
+      hipFuncSetAttribute(reinterpret_cast<const void*>(nvfp4_prefill_kernel<false>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)PV_SMEM),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(nvfp4_prefill_kernel<true>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)PV_SMEM)};
+  if (attr[pipe] != hipSuccess) return -6;
+  hipLaunchKernelGGL(pipe ? nvfp4_prefill_kernel<true> : nvfp4_prefill_kernel<false>, grid, dim3(PV_THREADS), PV_SMEM,
+                     (hipStream_t)stream, (const uint8_t*)a, (const float*)as, (const uint8_t*)wq, (const uint8_t*)ws,
+                     (const float*)wg, (uint16_t*)c, (const int*)sorted_ids, (const int*)expert_ids,
+                     (const int*)ntpp, (const float*)topk_w, wq_estride, ws_estride, wg_estride, numel, a_row_div, K, N,
+                     blk, subs);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 

@@ -117,6 +117,26 @@ def test_nvfp4_linear_prefill_k_tiles(dev, M, N, Kd):
     test_nvfp4_linear(dev, M, N, Kd)
 
 
+@pytest.mark.parametrize("M,N,Kd", [(129, 144, 128), (4096, 4096, 320), (4100, 4112, 512), (2000, 8192, 416)])
+def test_nvfp4_linear_prefill_short_k(dev, M, N, Kd):
+    """The loop without the software pipeline: one K-tile, and three or four K-tiles over 1024 tiles and more. Rows at both
+    ends of the row blocks and spread columns against the pipelined loop's bits (fewer rows of the same input) and the
+    oracle."""
+    g = torch.Generator().manual_seed(20261201 + 4700 + M + N + Kd)
+    packed, s16, wg = make_nv(1, N, Kd, g)
+    W = K.prepare_nvfp4_weights(packed.to(dev), s16.to(dev), wg.to(dev))
+    x = torch.randn(M, Kd, generator=g).to(torch.bfloat16)
+    out = ops.nvfp4_linear(x.to(dev), W.wq, W.ws, W.wg, N, Kd)
+    rows = torch.cat([torch.arange(0, 65), torch.arange(M - 64, M)])          # 129 rows: two row blocks
+    few = ops.nvfp4_linear(x[rows].to(dev), W.wq, W.ws, W.wg, N, Kd)
+    torch.cuda.synchronize()
+    assert torch.equal(out.cpu()[rows].view(torch.int16), few.cpu().view(torch.int16))
+    qo, so = O.quant_rows_fp8(x[rows])
+    ref = O.nvfp4_gemm(qo, so, packed.numpy(), s16.view(torch.uint8).numpy(), wg.numpy(),
+                       np.zeros(len(rows), dtype=np.int32), 1)
+    check(O.bf16_bits(few), ref)
+
+
 @pytest.mark.parametrize("M", [31, 32, 33, 64, 65, 127])
 def test_nvfp4_linear_wide_decode_blocks(dev, M):
     """Long K (5 K-tiles and more a wave) at 32- and 64-row routing blocks, where at most two blocks are launched."""
