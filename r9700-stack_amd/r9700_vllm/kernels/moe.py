@@ -992,6 +992,19 @@ def dense_nvfp4_qa(x: torch.Tensor, w: Nvfp4Experts, out: torch.Tensor) -> bool:
 DENSE_NV_A8_MAX_M = int(os.environ.get("R9K_DENSE_NV_A8_MAX_M", "16"))
 
 
+def dense_nvfp4_a8_wanted(M: int, N: int, K: int) -> bool:
+    """Whether a native NVFP4 linear of quantised rows takes the dense kernel. It runs a workgroup a column tile, six a CU:
+    of short K, whose workgroups end together, a last round of them that leaves a third of the chip idle or more costs
+    more from 13 rows on than the tables. Measured on MI355X at 16 rows, K = 1024, decode kernel -> dense kernel, us: N =
+    32768 (1 1/3 rounds) 8.0 -> 9.3, 40960 (1 2/3) 9.1 -> 10.2, 65536 (2 2/3) 12.9 -> 14.0, 45056 (1 5/6) 10.5 -> 9.7, 49152
+    (2) 11.5 -> 10.7, 24576 (1) 7.0 -> 6.6; K = 1152, N = 32768 9.2 -> 9.9, K = 1280 and more even or faster, K = 512 (one
+    wave a workgroup) faster."""
+    if M > DENSE_NV_A8_MAX_M:
+        return False
+    left = N // 16 % 1536
+    return not (M >= 13 and 1024 <= K <= 1152 and N > 16 * 1536 and 0 < left <= 1024)
+
+
 def dense_nvfp4_a8(q: torch.Tensor, s: torch.Tensor, w: Nvfp4Experts, out: torch.Tensor) -> bool:
     """out [M, N] = bf16(dequant(q, s) @ W^T) for one native NVFP4 weight and M <= 16 rows already quantised
     (quant_rows_fp8's codes and scales), without routing tables (r9k_dense_nvfp4_a8): the values of moe_gemm over

@@ -121,7 +121,7 @@ def _nvfp4_linear_rows(x: torch.Tensor, W, out: torch.Tensor) -> None:
     if M <= KM.DENSE_NV_QA_MAX_M and KM.dense_nvfp4_qa(x, W, out):   # decode widths: the quant inside the GEMM launch
         return
     q, s = KM.quant_rows_fp8(x)
-    if M <= KM.DENSE_NV_A8_MAX_M and KM.dense_nvfp4_a8(q, s, W, out):
+    if KM.dense_nvfp4_a8_wanted(M, W.N, W.K) and KM.dense_nvfp4_a8(q, s, W, out):
         return
     if M >= KM.NV_PREFILL_MIN_M and W.K % 32 == 0:
         tabs = IdentityTables.get(x.device, M, KM.prefill_block(KM.NV_PREFILL_CFG))

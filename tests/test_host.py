@@ -229,6 +229,15 @@ def test_tuned_table_lookup(tmp_path, monkeypatch):
     monkeypatch.setattr(tuned, "_TABLE", None)
 
 
+@pytest.mark.parametrize("N,Kd,first", [
+    (32768, 1024, 13), (28672, 1024, 13), (40960, 1024, 13), (65536, 1024, 13), (32768, 1152, 13),
+    (24576, 1024, 17), (45056, 1024, 17), (49152, 1024, 17), (32768, 1280, 17), (32768, 2048, 17), (65536, 512, 17),
+    (17408, 5120, 17), (1024, 1024, 17)])
+def test_native_nvfp4_dense_width(N, Kd, first):
+    """Rows from which a native NVFP4 linear leaves the dense kernel, over shapes timed on both."""
+    assert [K.dense_nvfp4_a8_wanted(m, N, Kd) for m in range(1, 20)] == [m < first for m in range(1, 20)]
+
+
 def test_apply_chunks_end_at_one_token(monkeypatch):
     """A step past the buffer limit runs as its chunks, and a chunk of one token runs whatever its size."""
     import r9700_vllm.moe.experts as X
