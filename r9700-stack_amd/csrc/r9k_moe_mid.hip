@@ -7,20 +7,24 @@
 //
 // What bounds it: at these widths a routing block's weights are used for 16-128 rows, so the launch is a weight
 // stream (HBM) with the activation rows re-read from L2 by every column block; a workgroup's steps are bounded by the
-// global -> LDS path (64 bytes a clock a CU: 270 clocks for 64 x 128) and, beside it, by the waves' instruction count.
-// The decode kernel it replaces here read both operands into registers with no reuse across waves and nothing in
-// flight during its MFMAs. Measured on MI355X, before -> after: routed gate_up [640, 2560] x 512 experts, top-10, 3001
-// tokens 243 -> 124 us, down [2560, 320] 244 -> 97 (220 MB of weights and 154 MB out: 3.9 TB/s); dense [17408, 5120] at
-// 37 / 64 / 333 rows 23.2 / 36 / 125 -> 14.9 / 15.4 / 33 us (64 rows: 3.1 TB/s of weights; 333 rows: 1.8 PFLOP/s);
-// dense [4096, 4096] at 1024 rows, from the 256-row kernel, 44 -> 20 us.
+// global -> LDS path (64 bytes a clock a CU: 270 clocks for 64 x 128) and, beside it, by the waves' instruction count;
+// from a few hundred rows by the MFMAs and by tiles that do not divide into whole rounds of the CUs. The decode kernel
+// it replaces here read both operands into registers with no reuse across waves and nothing in flight during its MFMAs.
+// Measured on MI355X, before -> after: routed gate_up [640, 2560] x 512 experts, top-10, 3001 tokens 243 -> 124 us, down
+// [2560, 320] 244 -> 97 (220 MB of weights and 154 MB out: 3.9 TB/s); dense [17408, 5120] at 36 / 64 / 333 rows, weights
+// cold in every cache, 24.5 / 37.7 / 126 -> 17.9 / 20.1 / 39 us, and 23.2 / 36 / 125 -> 14.9 / 15.4 / 33 with them in the
+// 256 MB last-level cache (64 rows: 2.4 and 3.1 TB/s of weights; 333 rows: 1.5 and 1.8 PFLOP/s); dense [4096, 4096] at
+// 1024 rows, from the 256-row kernel, 44 -> 20 us.
 //
-// Work split: a workgroup of 2 x WN waves (per K group) owns BM rows x BN columns, and walks `span` consecutive column blocks of
-// its routing block. The (column block, 128-wide K chunk) steps run as one stream through a ring of NS LDS stages
-// filled by direct global -> LDS DMA, NS - 1 steps ahead, across the column blocks' boundaries; where the tiles fill
-// the chip, two workgroups a CU (at most 80 KB of LDS each) cover each other's table reads and epilogues; where they do
-// not, KS groups of waves in one workgroup split the K chunks and their partial sums meet in LDS, in group order. Each step every thread issues OPS DMA
-// loads; an explicit vmcnt wait plus a barrier publishes the stage. The loop holds no compiler-tracked global load, so
-// nothing else drains the ring, and each column block's ST output stores are counted in the waits of the steps after.
+// Work split: a workgroup of 2 x WN waves (per K group) owns BM rows x BN columns, and walks `span` consecutive column
+// blocks of its routing block. The (column block, 128-wide K chunk) steps run as one stream through a ring of NS LDS
+// stages filled by direct global -> LDS DMA, NS - 1 steps ahead, across the column blocks' boundaries. Where the tiles
+// fill the chip, two workgroups of 256 threads a CU (at most 80 KB of LDS each) cover each other's table reads and
+// epilogues, except in the 256-column variant for short K: 512 threads and 83.75 KB, one a CU, where halving the
+// activation re-reads is worth more. Where they do not, KS groups of waves in one workgroup split the K chunks and their
+// partial sums meet in LDS, in group order. Each step every thread issues OPS DMA loads; an explicit vmcnt wait plus a
+// barrier publishes the stage. The loop holds no compiler-tracked global load, so nothing else drains the ring, and each
+// column block's ST output stores are counted in the waits of the steps after.
 //
 // Operands of V_MFMA_SCALE_F32_16X16X128_F8F6F4 (layout measured on gfx950, see r9k_moe_gemm.hip): the weights in the A
 // slot (fp4, their e8m0 exponent as the A scale), the activations in the B slot (fp8, scale 2^0). A lane of the result
@@ -59,6 +63,7 @@ struct Mid {
   static constexpr int ST = MTW * CT / 2;                      // output stores a wave and column block
   static constexpr size_t SMEM = (size_t)NS * STAGE + NW * 1024;
   static_assert(SMEM <= 160 * 1024 && NS >= 3 && MA >= 1, "LDS");
+  static_assert(KS > 1 || NW > 4 || SMEM <= 80 * 1024, "two workgroups of 256 threads a CU");
   static_assert((KS - 1) * NW * MTW * CT * 1024 <= NS * STAGE, "partial sums fit the ring");
   static_assert((NS - 1) * OPS + ST < 64, "vmcnt");
 };

@@ -666,9 +666,8 @@ __global__ void __launch_bounds__(WAVE * SK) dense_nvfp4_qa_kernel(
 // The native NVFP4 dense linear for M <= 16 rows already quantised: moe_nvfp4_kernel's weight stream for one routing
 // block of identity rows without the tables -- the same widening, MFMA order, K split over SK waves and partial-tile
 // sum, so the same bits. Bound by the weight bytes and the widening's issue slots. Against that kernel over identity
-// tables it starts its weight loads with its first instructions (no ntpp -> expert -> row id chain before them),
-// launches no workgroups for a second, empty block, and refills a K-tile's registers as soon as the tile is widened
-// instead of draining a batch before the next. One column tile a workgroup and two K-tiles in flight a wave: 80
+// tables it starts its weight loads with its first instructions (no ntpp -> expert -> row id chain before them) and
+// refills a K-tile's registers as soon as the tile is widened instead of draining a batch before the next. One column tile a workgroup and two K-tiles in flight a wave: 80
 // registers, six waves a SIMD, which hide more than a deeper ring on fewer waves (MI355X, GEMM alone, [17408, 5120] at
 // M = 4: 14.2 us; 3 tiles 15.2, 4 15.2, 5 15.5, 10 16.1). Decode kernel -> this one, us: [17408, 5120] M = 4 / 8 / 16
 // 16.1 / 17.9 / 20.3 -> 14.2 / 15.0 / 18.3, [5120, 17408] 22.4 / 23.5 / 27.0 -> 19.2 / 18.9 / 21.9, [4096, 4096]

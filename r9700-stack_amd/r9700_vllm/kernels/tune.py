@@ -3,7 +3,8 @@
     python -m r9700_vllm.kernels.tune [--out PATH] [--reps 20]
 
 For each dense product (N, K) in SHAPES and each row count M in MS (the rows between the dense weight stream's 16 and
-the prefill kernel's 128, where ops.mxfp4_gemm_q runs r9k_moe_mxfp4a8 over identity tables), every built launch
+the prefill kernel's 128) at which ops.mxfp4_gemm_q runs r9k_moe_mxfp4a8 over identity tables, and not the LDS-ring
+kernel (kernels.moe.dense_mid_wanted; with R9K_DENSE_MID=0 all of them), every built launch
 shape (WV, SK, NPW in {1, 2, 4}, those legal_cfg accepts) and the kernel's own choice (0, 0, 0) are timed: a HIP
 graph of `reps` launches cycling through enough weight copies to exceed the 256 MB Infinity Cache, HIP events around
 its replay. The fastest shape is written with its time and the kernel's own choice's, so the table records how much
@@ -19,7 +20,7 @@ import sys
 
 import torch
 
-SHAPES = ((1024, 2048), (17408, 5120), (2048, 2048), (4096, 4096))
+SHAPES = ((1024, 2048), (17408, 5120), (2048, 2048), (4096, 4096))      # [17408, 5120] only with R9K_DENSE_MID=0
 MS = (17, 24, 32, 48, 64, 96, 127)
 
 
@@ -78,7 +79,7 @@ def main(argv=None) -> int:
         return 1
     entries = []
     for N, K in SHAPES:
-        for M in MS:
+        for M in (m for m in MS if not KM.dense_mid_wanted(m, N, K)):
             cands = [(0, 0, 0)] + [c for c in itertools.product(KM.BUILT_KNOBS, repeat=3)
                                    if KM.legal_cfg(c, N, K, MT=KM.decode_mt(M)) == c]
             res = time_shape(N, K, M, cands, args.reps)

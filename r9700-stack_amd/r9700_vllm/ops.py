@@ -1,14 +1,15 @@
-"""torch.library custom ops over libr9k's ctypes kernels, so the dense linears can sit inside a torch.compile'd
-graph (Dynamo cannot trace a ctypes call) and be captured into HIP graphs. The reference's r9700_vllm/ops.py surface
+"""torch.library custom ops over libr9k's entries, so the dense linears can sit inside a torch.compile'd
+graph (Dynamo cannot trace a call into the library) and be captured into HIP graphs. The reference's r9700_vllm/ops.py surface
 for the 4-bit path:
 
   torch.ops.r9700.mxfp4_linear(x [M, K] bf16, wq, wsr, N, K, fold) -> [M, N] bf16   MXFP4 weight, per-token fp8 act
   torch.ops.r9700.nvfp4_linear(x [M, K] bf16, wq, ws, wg, N, K) -> [M, N] bf16      native NVFP4 weight (exact bits)
 
 plus `mxfp4_gemm_q` (the GEMM on already-quantised rows, which the shared expert uses). A dense linear is the grouped
-MoE GEMM with one expert and identity routing tables (`IdentityTables`); at decode widths the MXFP4 linear is one
-launch with the activation quant inside (kernels.moe.dense_mxfp4_qa), and up to 16 rows the GEMM on quantised rows
-is the dense kernel's weight stream (kernels.moe.dense_mxfp4_a8). The reference's fp8_linear / fp8_block_linear
+MoE GEMM with one expert and identity routing tables (`IdentityTables`). At decode widths it is one launch with the
+activation quant inside (kernels.moe.dense_mxfp4_qa, dense_nvfp4_qa), then, up to 16 rows, the quant and the dense
+kernel's weight stream without tables (dense_mxfp4_a8, dense_nvfp4_a8); wide MXFP4 linears leave these from 12 rows on
+for the LDS-ring kernel (kernels.moe.dense_mid_wanted). The reference's fp8_linear / fp8_block_linear
 (dense fp8 GEMMs) are outside this build.
 """
 from __future__ import annotations
@@ -135,8 +136,9 @@ def _nvfp4_linear_rows(x: torch.Tensor, W, out: torch.Tensor) -> None:
 def _nvfp4_linear(x: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, wg: torch.Tensor, N: int, K: int
                   ) -> torch.Tensor:
     """Native NVFP4 weights (prepare_nvfp4_weights of one expert) with per-row fp8 activations: one launch with the
-    quant inside up to DENSE_NV_QA_MAX_M rows, the decode-family kernel below NV_PREFILL_MIN_M rows, the 128 x 128-tile
-    prefill kernel (r9k_moe_4bit_prefill nv = 1) from there; row ranges past the 2 GiB buffer range (row_ranges)."""
+    quant inside up to DENSE_NV_QA_MAX_M rows, the quant and the table-less dense kernel up to DENSE_NV_A8_MAX_M
+    (dense_nvfp4_a8_wanted), the decode-family kernel below NV_PREFILL_MIN_M rows, the 128 x 128-tile prefill kernel
+    (r9k_moe_4bit_prefill nv = 1) from there; row ranges past the 2 GiB buffer range (row_ranges)."""
     M = x.shape[0]
     out = KM._empty(x, torch.bfloat16, M, N)
     W = KM.Nvfp4Experts(wq, ws, wg, N, K)

@@ -890,10 +890,14 @@ def test_decode_gemm_reference_knobs_ignored(dev, MT):
         assert np.array_equal(run(*knobs), auto), knobs
 
 
-@pytest.mark.parametrize("M,N,Kd", [(17, 1024, 2048), (40, 1024, 2048), (100, 1024, 2048), (48, 17408, 5120)])
+@pytest.mark.parametrize("M,N,Kd", [(17, 1024, 2048), (40, 1024, 2048), (63, 1024, 2048), (32, 4096, 4096),
+                                    (100, 1024, 2048), (48, 17408, 5120)])
 def test_dense_linear_tuned_shapes(dev, M, N, Kd):
     """ops.mxfp4_linear between the dense weight stream's 16 rows and the prefill kernel's 128: the decode kernel at
-    the launch table's shape (kernels/tuned.json), against the oracle on 24 sampled rows."""
+    the launch table's shape (kernels/tuned.json), or the LDS-ring kernel at the last two widths, against the oracle on
+    24 sampled rows."""
+    ring = K.dense_mid_wanted(M, N, Kd)
+    assert ring == (M in (100, 48)) and (ring or 0 not in K.pick_cfg(N, Kd, M=M, kind="mxfp4"))
     g = torch.Generator().manual_seed(20261201 + 22000 + M + N)
     packed, e8 = make_experts(1, N, Kd, g)
     W = K.prepare_mxfp4_weights(packed.to(dev), e8.to(dev))

@@ -272,6 +272,15 @@ def test_conversion_launch_rows():
         assert _launch_rows(a, b, cpu, 2048) == 2048
 
 
+def test_every_launch_table_entry_is_looked_up():
+    """pick_cfg answers with each entry of the committed table at its own width (none is shadowed by another kernel)."""
+    from r9700_vllm.kernels import tuned
+    assert len(tuned.table()["entries"]) >= 8
+    for e in tuned.table()["entries"]:
+        got = K.pick_cfg(e["N"], e["K"], M=e["M"], kind=e["kind"])
+        assert got == tuple(e["cfg"]), (e, got)
+
+
 @pytest.fixture
 def entry(monkeypatch):
     """A stand-in for a libr9k entry behind kernels.moe._call: records its four C arguments (long, long, int, long)."""
