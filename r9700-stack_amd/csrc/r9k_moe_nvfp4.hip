@@ -667,11 +667,12 @@ __global__ void __launch_bounds__(WAVE * SK) dense_nvfp4_qa_kernel(
 // block of identity rows without the tables -- the same widening, MFMA order, K split over SK waves and partial-tile
 // sum, so the same bits. Bound by the weight bytes and the widening's issue slots. Against that kernel over identity
 // tables it starts its weight loads with its first instructions (no ntpp -> expert -> row id chain before them) and
-// refills a K-tile's registers as soon as the tile is widened instead of draining a batch before the next. One column tile a workgroup and two K-tiles in flight a wave: 80
-// registers, six waves a SIMD, which hide more than a deeper ring on fewer waves (MI355X, GEMM alone, [17408, 5120] at
-// M = 4: 14.2 us; 3 tiles 15.2, 4 15.2, 5 15.5, 10 16.1). Decode kernel -> this one, us: [17408, 5120] M = 4 / 8 / 16
-// 16.1 / 17.9 / 20.3 -> 14.2 / 15.0 / 18.3, [5120, 17408] 22.4 / 23.5 / 27.0 -> 19.2 / 18.9 / 21.9, [4096, 4096]
-// 7.3 / 7.5 / 10.4 -> 6.6 / 6.5 / 7.0, [1024, 2048] 6.0 / 6.1 / 6.5 -> 4.6 / 4.7 / 4.9.
+// refills a K-tile's registers as soon as the tile is widened instead of draining a batch before the next. One
+// column tile a workgroup and two K-tiles in flight a wave: 80 registers, six waves a SIMD, which hide more than a
+// deeper ring on fewer waves (MI355X, GEMM alone, [17408, 5120] at M = 4: 14.2 us; 3 tiles 15.2, 4 15.2, 5 15.5, 10
+// 16.1). Decode kernel -> this one, us: [17408, 5120] M = 4 / 8 / 16 16.1 / 17.9 / 20.3 -> 14.2 / 15.0 / 18.3,
+// [5120, 17408] 22.4 / 23.5 / 27.0 -> 19.2 / 18.9 / 21.9, [4096, 4096] 7.3 / 7.5 / 10.4 -> 6.6 / 6.5 / 7.0, [1024,
+// 2048] 6.0 / 6.1 / 6.5 -> 4.6 / 4.7 / 4.9.
 template <int SK>
 __global__ void __launch_bounds__(WAVE * SK) dense_nvfp4_a8_kernel(
     const uint8_t* __restrict__ A, long lda, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
