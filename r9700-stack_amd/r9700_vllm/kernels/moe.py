@@ -679,9 +679,9 @@ DEVICE_MIN_ROWS = int(os.environ.get("R9K_MOE_DEVICE_MIN_ROWS", "22"))
 
 # Routed steps of small experts (gate_up codes below MID_MAX_BYTES) run on 64-row blocks of the LDS-ring kernel from
 # MID_MIN_ROWS rows an expert: a 64-row block streams its expert's weights once, so experts with a handful of rows
-# cost little more than their weights. Measured on MI355X over 23 layers (0.2 to 3.9 MB of gate_up codes an expert, 16
+# cost little more than their weights. Measured on MI355X over 22 layers (0.2 to 3.8 MB of gate_up codes an expert, 16
 # to 512 experts) under uniform, Zipf(0.6) and Zipf(1.1) routing, against decode blocks, split tables or 256-row
-# blocks, whichever such a step takes without this: geometric mean of the whole layer's time 0.81 at 10 rows, 0.78 at
+# blocks, whichever such a step takes without this: geometric mean of the whole layer's time 0.84 at 10 rows, 0.73 at
 # 48. A down product whose K fills its 128-wide tiles by three quarters or less (K = 160, 192) starts at MID_MIN_ROWS
 # + 2: 128 experts, hidden 4096, intermediate 192 at 10 / 12 rows 68.8 -> 74.3, 74.8 -> 74.1 us. Where a K is not a
 # multiple of 128, 128-row blocks follow from MID_ODD_ROWS: 512 experts, hidden 2560, intermediate 320 at 64 / 72 / 96
@@ -690,7 +690,7 @@ DEVICE_MIN_ROWS = int(os.environ.get("R9K_MOE_DEVICE_MIN_ROWS", "22"))
 # more than they save while the layer is small: 288 experts, hidden 2048, intermediate 512, uniform / Zipf(0.6) /
 # Zipf(1.1), us: 72 rows 243 / 260 / 193 split, 225 / 224 / 189 on 64-row blocks, 225 / 272 / 204 on 256-row ones; 96
 # rows 264 / 284 / 228, 248 / 253 / 230 and 243 / 294 / 224. A layer of MID_SPLIT_BYTES gate_up codes and more keeps
-# its split tables, from MID_SPLIT_ROWS: 256 experts, hidden 3072, intermediate 1024 on 256-row blocks 0.96 / 1.09 /
+# its split tables, from MID_SPLIT_ROWS: 256 experts, hidden 3072, intermediate 1024 on 256-row blocks 1.00 / 1.09 /
 # 1.14 of the split tables' time at 80 rows, 0.96 / 1.06 / 1.09 at 128 (512 experts, hidden 2048, intermediate 1024 at
 # 72 0.98 / 1.19 / 1.10); on 64-row blocks 0.96 / 0.95 / 1.03 at 64 rows, 1.06 / 0.97 / 1.05 at 80.
 # R9K_MOE_MID=0 turns all of it off, and so does setting a variable that chooses these steps' blocks itself.
